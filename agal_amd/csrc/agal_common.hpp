@@ -398,6 +398,14 @@ struct Store<float, bf16s> {
     static constexpr bool quantized = true;
 };
 
+// Orders a wavefront's LDS accesses: what its lanes wrote before is seen by what they read after.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The value a store followed by a load yields.
 template <typename T, typename S>
 __device__ __forceinline__ T quant(T f, T w)

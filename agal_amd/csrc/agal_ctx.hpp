@@ -39,8 +39,10 @@ struct Predictor {
     float *snap = nullptr;  // feature snapshots, snap_slots x n_maxcblocks x NFEAT
     int snap_slots = 0;
     int batch_cap = 0;      // rows of the training buffers below
-    float *X = nullptr, *Y = nullptr, *Z1 = nullptr, *Z2 = nullptr, *z3 = nullptr, *dZ3 = nullptr, *dZ2 = nullptr,
-          *dZ1 = nullptr, *loss = nullptr;
+    long long batch_ld = 0;  // row length of the transposed buffers XT (features) and H1T (hidden layer 1)
+    float *X = nullptr, *Y = nullptr, *XT = nullptr, *H1T = nullptr, *H2 = nullptr, *z3 = nullptr, *dZ3 = nullptr,
+          *dZ2 = nullptr, *dZ1 = nullptr, *loss = nullptr;
+    double *loss_sum = nullptr;
     int *ids = nullptr;
 };
 
@@ -252,7 +254,7 @@ void predictor_init_weights(unsigned long long seed, float *w);
 int predictor_setup(Ctx *c, unsigned long long seed, int batch_cap);
 int predictor_set_weights(Ctx *c, const float *w_host);
 int predictor_get(Ctx *c, int which, float *out);
-int predictor_forward_dev(Ctx *c, const float *X, int n, float *z3, float *p, float *Z1, float *Z2);
+int predictor_forward_dev(Ctx *c, const float *X, int n, float *z3, float *p);
 int predictor_train_dev(Ctx *c, int n, float lr, float pos_weight, double *loss);
 int predictor_features(Ctx *c);
 int predictor_predict_blocks(Ctx *c);

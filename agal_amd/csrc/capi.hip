@@ -1235,7 +1235,7 @@ int agal_predictor_forward(agal_ctx *ctx, const float *x, int n, float *z_out, f
     if (n < 0 || n > c->pred.batch_cap || (n > 0 && !x)) return AGAL_ERR_ARG;
     if (n == 0) return AGAL_OK;
     AGAL_HIP(c, hipMemcpyAsync(c->pred.X, x, sizeof(float) * NFEAT * n, hipMemcpyHostToDevice, c->stream));
-    int st = predictor_forward_dev(c, c->pred.X, n, c->pred.z3, c->pred.Y, nullptr, nullptr);
+    int st = predictor_forward_dev(c, c->pred.X, n, c->pred.z3, c->pred.Y);
     if (st) return st;
     if (z_out) AGAL_HIP(c, hipMemcpyAsync(z_out, c->pred.z3, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
     if (p_out) AGAL_HIP(c, hipMemcpyAsync(p_out, c->pred.Y, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));

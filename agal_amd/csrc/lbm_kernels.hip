@@ -312,13 +312,6 @@ __constant__ const MfmaTab<27> kMfma27 = make_mfma_tab<27>();
 
 constexpr int MFMA_SPLITS = 2;
 
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Next bf16 term of `rem` (round to nearest even, the hardware conversion); rem keeps the rest.
 __device__ __forceinline__ __bf16 split_term(float &rem)
 {

@@ -203,120 +203,222 @@ __global__ void k_features(int id_max, const int *__restrict__ ref, const int *_
 }
 
 // ---------------------------------------------------------------------------------------------
-// The network.  Weights are staged in LDS as FP32 values of the FP16 copy; one thread per sample.
+// The network.  One wavefront takes groups of four rows; lane j is hidden unit j of both layers and
+// keeps its column of W1 and W2 (for the backward pass also its row of W2) in registers, converted
+// once from the FP16 copy; activations go from lane to lane through LDS as broadcast 16-byte reads
+// that serve four products each.  Each dot product is one lane's chain in index order.  A batch is
+// latency bound (4096 rows are 1024 wavefronts of one group each): 4096 rows took 52 us forward and
+// 62 us backward with one thread per row, 64 wavefronts, and each weight read from LDS per product.
 // ---------------------------------------------------------------------------------------------
-__device__ inline void stage_weights(const _Float16 *__restrict__ wh, float *s_w)
-{
-    for (int q = threadIdx.x; q < MLP_NPARAM; q += blockDim.x) s_w[q] = (float)wh[q];
-    __syncthreads();
-}
-
 __device__ inline float sigmoidf_dev(float z) { return 1.0f / (1.0f + expf(-z)); }
 
-// Forward pass over n feature rows; optional outputs z1, z2 (n x 64) for training.
-__global__ __launch_bounds__(PWG) void k_mlp_forward(const float *__restrict__ X, int n, const _Float16 *__restrict__ wh,
-                                                     float *__restrict__ z3_out, float *__restrict__ p_out,
-                                                     float *__restrict__ Z1, float *__restrict__ Z2)
-{
-    __shared__ float s_w[MLP_NPARAM];
-    stage_weights(wh, s_w);
-    const int r = blockIdx.x * PWG + threadIdx.x;
-    if (r >= n) return;
-    const float *W1 = s_w + MLP_OFF_W1, *B1 = s_w + MLP_OFF_B1, *W2 = s_w + MLP_OFF_W2, *B2 = s_w + MLP_OFF_B2;
-    const float *W3 = s_w + MLP_OFF_W3;
-    float x[NFEAT];
-    for (int i = 0; i < NFEAT; i++) x[i] = X[(long long)NFEAT * r + i];
-    float h1[MLP_H];
-    for (int j = 0; j < MLP_H; j++) {
-        float z = B1[j];
-        for (int i = 0; i < NFEAT; i++) z += x[i] * W1[i * MLP_H + j];
-        if (Z1) Z1[(long long)MLP_H * r + j] = z;
-        h1[j] = z > 0.f ? z : 0.f;
-    }
-    float z3 = s_w[MLP_OFF_B3];
-    for (int k = 0; k < MLP_H; k++) {
-        float z = B2[k];
-        for (int j = 0; j < MLP_H; j++) z += h1[j] * W2[j * MLP_H + k];
-        if (Z2) Z2[(long long)MLP_H * r + k] = z;
-        z3 += (z > 0.f ? z : 0.f) * W3[k];
-    }
-    if (z3_out) z3_out[r] = z3;
-    if (p_out) p_out[r] = sigmoidf_dev(z3);
-}
+constexpr int MLP_R = 4;          // rows per wavefront and pass
+constexpr int MLP_LD = MLP_H + 4;  // LDS row stride: the four rows' 16-byte reads fall in distinct banks
 
-// Loss and output gradient of the weighted binary cross-entropy on logits:
+// What the parameter gradients need of each row; lengths of the transposed arrays' rows: ld (a
+// multiple of MLP_R, at least the batch).
+struct MlpTrain {
+    const float *Y;
+    float pos_weight;
+    long long ld;
+    float *XT, *H1T;             // features and h1, one array of rows per feature / unit
+    float *H2, *dZ2, *dZ1;       // n x 64
+    float *dZ3, *loss;           // n
+};
+
+// Forward pass over n feature rows.  TRAIN: also the weighted binary cross-entropy on logits and the
+// deltas of every layer,
 //   loss_r = w_r (y_r softplus(-z) + (1 - y_r) softplus(z)),  w_r = pos_weight if y_r = 1 else 1,
-//   dL/dz_r = w_r (sigmoid(z) - y_r) / n.
-__global__ void k_mlp_output_grad(const float *__restrict__ z3, const float *__restrict__ Y, int n, float pos_weight,
-                                  float *__restrict__ dZ3, float *__restrict__ loss)
+//   dL/dz_r = w_r (sigmoid(z) - y_r) / n,
+//   dz2_k = dz3 W3_k [z2_k > 0],  dz1_j = [z1_j > 0] sum_k W2_jk dz2_k.
+template <bool TRAIN>
+__global__ __launch_bounds__(PWG) void k_mlp_rows(const float *__restrict__ X, int n, const _Float16 *__restrict__ wh,
+                                                  float *__restrict__ z3_out, float *__restrict__ p_out, MlpTrain tr)
 {
-    const int r = blockIdx.x * PWG + threadIdx.x;
-    if (r >= n) return;
-    const float z = z3[r], y = Y[r];
-    const float wgt = y > 0.5f ? pos_weight : 1.0f;
-    const float sp_pos = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z)));  // softplus(z)
-    const float sp_neg = sp_pos - z;                                // softplus(-z)
-    loss[r] = wgt * (y * sp_neg + (1.0f - y) * sp_pos);
-    dZ3[r] = wgt * (sigmoidf_dev(z) - y) / (float)n;
+    typedef __attribute__((ext_vector_type(4))) float f4;
+    __shared__ __attribute__((aligned(16))) float s_all[PWG / 64][2 * MLP_R * MLP_LD];
+    __shared__ __attribute__((aligned(16))) float s_xall[PWG / 64][MLP_R * NFEAT];
+    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    float *s_h = s_all[wv], *s_t = s_h + MLP_R * MLP_LD, *s_x = s_xall[wv];
+    float w1[NFEAT], w2[MLP_H], w2r[TRAIN ? MLP_H : 1];
+#pragma unroll
+    for (int i = 0; i < NFEAT; i++) w1[i] = (float)wh[MLP_OFF_W1 + i * MLP_H + l];
+#pragma unroll
+    for (int j = 0; j < MLP_H; j++) w2[j] = (float)wh[MLP_OFF_W2 + j * MLP_H + l];
+    if constexpr (TRAIN) {
+#pragma unroll
+        for (int k = 0; k < MLP_H; k++) w2r[k] = (float)wh[MLP_OFF_W2 + l * MLP_H + k];
+    }
+    const float b1 = (float)wh[MLP_OFF_B1 + l], b2 = (float)wh[MLP_OFF_B2 + l], w3 = (float)wh[MLP_OFF_W3 + l];
+    const float b3 = (float)wh[MLP_OFF_B3];
+    const long long step = (long long)gridDim.x * (PWG / 64) * MLP_R;
+    for (long long r0 = ((long long)blockIdx.x * (PWG / 64) + wv) * MLP_R; r0 < n; r0 += step) {
+        if (l < MLP_R * NFEAT) s_x[l] = NFEAT * r0 + l < (long long)NFEAT * n ? X[NFEAT * r0 + l] : 0.f;
+        wave_lds_sync();
+        float z1[MLP_R], z2[MLP_R];
+#pragma unroll
+        for (int r = 0; r < MLP_R; r++) {
+            float z = b1;
+#pragma unroll
+            for (int i = 0; i < NFEAT; i++) z += s_x[r * NFEAT + i] * w1[i];
+            z1[r] = z;
+            s_h[r * MLP_LD + l] = z > 0.f ? z : 0.f;
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int r = 0; r < MLP_R; r++) {
+            float z = b2;
+#pragma unroll
+            for (int j = 0; j < MLP_H; j += 4) {
+                const f4 h = *reinterpret_cast<const f4 *>(s_h + r * MLP_LD + j);
+#pragma unroll
+                for (int e = 0; e < 4; e++) z += h[e] * w2[j + e];
+            }
+            z2[r] = z;
+            s_t[r * MLP_LD + l] = (z > 0.f ? z : 0.f) * w3;
+        }
+        wave_lds_sync();
+        // Lane l sums row l mod 4.
+        const int rl = l % MLP_R;
+        float z3 = b3;
+#pragma unroll
+        for (int k = 0; k < MLP_H; k += 4) {
+            const f4 t = *reinterpret_cast<const f4 *>(s_t + rl * MLP_LD + k);
+#pragma unroll
+            for (int e = 0; e < 4; e++) z3 += t[e];
+        }
+        const bool row = r0 + rl < n;
+        const float p = sigmoidf_dev(z3);
+        if (l < MLP_R && row) {
+            if (z3_out) z3_out[r0 + rl] = z3;
+            if (p_out) p_out[r0 + rl] = p;
+        }
+        if constexpr (TRAIN) {
+            float d3 = 0.f;
+            if (row) {
+                const float y = tr.Y[r0 + rl];
+                const float wgt = y > 0.5f ? tr.pos_weight : 1.0f;
+                const float sp_pos = fmaxf(z3, 0.f) + log1pf(expf(-fabsf(z3)));  // softplus(z)
+                const float sp_neg = sp_pos - z3;                                 // softplus(-z)
+                d3 = wgt * (p - y) / (float)n;
+                if (l < MLP_R) {
+                    tr.loss[r0 + rl] = wgt * (y * sp_neg + (1.0f - y) * sp_pos);
+                    tr.dZ3[r0 + rl] = d3;
+                }
+            }
+            float d2[MLP_R];
+            wave_lds_sync();  // the sums above have read s_t
+#pragma unroll
+            for (int r = 0; r < MLP_R; r++) {
+                const float d3r = __shfl(d3, r, 64);
+                d2[r] = z2[r] > 0.f ? d3r * w3 : 0.f;
+                s_t[r * MLP_LD + l] = d2[r];
+            }
+            wave_lds_sync();
+            f4 h1, x4;
+#pragma unroll
+            for (int r = 0; r < MLP_R; r++) {
+                float s = 0.f;
+#pragma unroll
+                for (int k = 0; k < MLP_H; k += 4) {
+                    const f4 d = *reinterpret_cast<const f4 *>(s_t + r * MLP_LD + k);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) s += w2r[k + e] * d[e];
+                }
+                h1[r] = z1[r] > 0.f ? z1[r] : 0.f;
+                x4[r] = l < NFEAT ? s_x[r * NFEAT + l] : 0.f;
+                if (r0 + r < n) {
+                    tr.dZ1[(r0 + r) * MLP_H + l] = z1[r] > 0.f ? s : 0.f;
+                    tr.dZ2[(r0 + r) * MLP_H + l] = d2[r];
+                    tr.H2[(r0 + r) * MLP_H + l] = z2[r] > 0.f ? z2[r] : 0.f;
+                }
+            }
+            *reinterpret_cast<f4 *>(tr.H1T + (long long)l * tr.ld + r0) = h1;
+            if (l < NFEAT) *reinterpret_cast<f4 *>(tr.XT + (long long)l * tr.ld + r0) = x4;
+        }
+        wave_lds_sync();  // s_x and s_h are read before the next group's
+    }
 }
 
-// Hidden-layer deltas per sample: dz2_k = dz3 W3_k [z2_k > 0]; dz1_j = [z1_j > 0] sum_k W2_jk dz2_k.
-__global__ __launch_bounds__(PWG) void k_mlp_backward(int n, const _Float16 *__restrict__ wh,
-                                                      const float *__restrict__ Z1, const float *__restrict__ Z2,
-                                                      const float *__restrict__ dZ3, float *__restrict__ dZ2,
-                                                      float *__restrict__ dZ1)
+// Parameter gradients: grad = sum over rows of S[r] V[r][lane], samples summed in order, one
+// wavefront per row of 64 parameters.  The row factor S is the same on every lane (scalar loads
+// from the transposed arrays); 64 rows of V are in flight while the 64 before them are summed, so
+// the wavefront runs near its chain of dependent adds (4096 rows: 1096 us with one thread per
+// parameter and a load per product in the chain).  The last wavefront sums the losses in FP64.
+constexpr int WG_ROWS = 64;
+
+template <bool HAS_S, bool HAS_V>
+__device__ __forceinline__ float wgrad_sum(int n, const float *__restrict__ S, const float *__restrict__ V, int l)
 {
-    __shared__ float s_w[MLP_NPARAM];
-    stage_weights(wh, s_w);
-    const int r = blockIdx.x * PWG + threadIdx.x;
-    if (r >= n) return;
-    const float *W2 = s_w + MLP_OFF_W2, *W3 = s_w + MLP_OFF_W3;
-    const float d3 = dZ3[r];
-    float d2[MLP_H];
-    for (int k = 0; k < MLP_H; k++) {
-        d2[k] = Z2[(long long)MLP_H * r + k] > 0.f ? d3 * W3[k] : 0.f;
-        dZ2[(long long)MLP_H * r + k] = d2[k];
+    float acc = 0.f;
+    float va[WG_ROWS], vb[WG_ROWS];
+    auto load = [&](float *v, int r) {
+        if constexpr (HAS_V) {
+#pragma unroll
+            for (int u = 0; u < WG_ROWS; u++) v[u] = V[(long long)(r + u) * MLP_H + l];
+        }
+    };
+    auto add = [&](const float *v, int r) {
+#pragma unroll
+        for (int u = 0; u < WG_ROWS; u++) {
+            if constexpr (HAS_S && HAS_V)
+                acc += S[r + u] * v[u];
+            else if constexpr (HAS_V)
+                acc += v[u];
+            else
+                acc += S[r + u];
+        }
+    };
+    const int full = n / WG_ROWS * WG_ROWS;
+    int r = 0;
+    if (full > 0) load(va, 0);
+    for (; r + 2 * WG_ROWS <= full; r += 2 * WG_ROWS) {
+        load(vb, r + WG_ROWS);
+        add(va, r);
+        if (r + 3 * WG_ROWS <= full) load(va, r + 2 * WG_ROWS);
+        add(vb, r + WG_ROWS);
     }
-    for (int j = 0; j < MLP_H; j++) {
-        float s = 0.f;
-        for (int k = 0; k < MLP_H; k++) s += W2[j * MLP_H + k] * d2[k];
-        dZ1[(long long)MLP_H * r + j] = Z1[(long long)MLP_H * r + j] > 0.f ? s : 0.f;
+    if (r < full) {
+        add(va, r);
+        r += WG_ROWS;
     }
+    for (; r < n; r++) {
+        const float v = HAS_V ? V[(long long)r * MLP_H + l] : 1.f;
+        acc += HAS_S && HAS_V ? S[r] * v : (HAS_V ? v : S[r]);
+    }
+    return acc;
 }
 
-// Parameter gradients, one thread per parameter, samples summed in order.
-__global__ void k_mlp_wgrad(int n, const float *__restrict__ X, const float *__restrict__ Z1,
-                            const float *__restrict__ Z2, const float *__restrict__ dZ3, const float *__restrict__ dZ2,
-                            const float *__restrict__ dZ1, float *__restrict__ grad)
+constexpr int WGRAD_WAVES = MLP_H + NFEAT + 5;
+
+__global__ __launch_bounds__(64) void k_mlp_wgrad(int n, long long ld, const float *__restrict__ XT,
+                                                  const float *__restrict__ H1T, const float *__restrict__ H2,
+                                                  const float *__restrict__ dZ3, const float *__restrict__ dZ2,
+                                                  const float *__restrict__ dZ1, const float *__restrict__ loss,
+                                                  float *__restrict__ grad, double *__restrict__ loss_sum)
 {
-    const int q = blockIdx.x * PWG + threadIdx.x;
-    if (q >= MLP_NPARAM) return;
-    float s = 0.f;
-    if (q < MLP_OFF_B1) {  // W1[i][j]
-        const int i = q / MLP_H, j = q % MLP_H;
-        for (int r = 0; r < n; r++) s += X[(long long)NFEAT * r + i] * dZ1[(long long)MLP_H * r + j];
-    } else if (q < MLP_OFF_W2) {  // b1[j]
-        const int j = q - MLP_OFF_B1;
-        for (int r = 0; r < n; r++) s += dZ1[(long long)MLP_H * r + j];
-    } else if (q < MLP_OFF_B2) {  // W2[j][k]
-        const int j = (q - MLP_OFF_W2) / MLP_H, k = (q - MLP_OFF_W2) % MLP_H;
-        for (int r = 0; r < n; r++) {
-            const float z = Z1[(long long)MLP_H * r + j];
-            s += (z > 0.f ? z : 0.f) * dZ2[(long long)MLP_H * r + k];
-        }
-    } else if (q < MLP_OFF_W3) {  // b2[k]
-        const int k = q - MLP_OFF_B2;
-        for (int r = 0; r < n; r++) s += dZ2[(long long)MLP_H * r + k];
-    } else if (q < MLP_OFF_B3) {  // W3[k]
-        const int k = q - MLP_OFF_W3;
-        for (int r = 0; r < n; r++) {
-            const float z = Z2[(long long)MLP_H * r + k];
-            s += (z > 0.f ? z : 0.f) * dZ3[r];
-        }
-    } else {  // b3
-        for (int r = 0; r < n; r++) s += dZ3[r];
+    const int l = threadIdx.x, b = blockIdx.x;
+    if (b < MLP_H) {
+        grad[MLP_OFF_W2 + b * MLP_H + l] = wgrad_sum<true, true>(n, H1T + b * ld, dZ2, l);
+    } else if (b < MLP_H + NFEAT) {
+        const int i = b - MLP_H;
+        grad[MLP_OFF_W1 + i * MLP_H + l] = wgrad_sum<true, true>(n, XT + i * ld, dZ1, l);
+    } else if (b == MLP_H + NFEAT) {
+        grad[MLP_OFF_B1 + l] = wgrad_sum<false, true>(n, nullptr, dZ1, l);
+    } else if (b == MLP_H + NFEAT + 1) {
+        grad[MLP_OFF_B2 + l] = wgrad_sum<false, true>(n, nullptr, dZ2, l);
+    } else if (b == MLP_H + NFEAT + 2) {
+        grad[MLP_OFF_W3 + l] = wgrad_sum<true, true>(n, dZ3, H2, l);
+    } else if (b == MLP_H + NFEAT + 3) {
+        const float s = wgrad_sum<true, false>(n, dZ3, nullptr, l);
+        if (l == 0) grad[MLP_OFF_B3] = s;
+    } else {
+        double s = 0;
+        for (int r = l; r < n; r += 64) s += loss[r];
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d, 64);
+        if (l == 0) *loss_sum = s;
     }
-    grad[q] = s;
 }
 
 // Adam (Kingma & Ba 2015) with bias correction; the FP16 copy follows the master weights.
@@ -405,7 +507,7 @@ void free_predictor(Ctx *c)
 {
     Predictor &P = c->pred;
     void *ptrs[] = {P.w, P.m, P.v, P.g, P.wh, P.stats, P.dist, P.feat, P.prob, P.label, P.snap, P.X, P.Y, P.ids,
-                    P.Z1, P.Z2, P.z3, P.dZ3, P.dZ2, P.dZ1, P.loss, P.counts};
+                    P.XT, P.H1T, P.H2, P.z3, P.dZ3, P.dZ2, P.dZ1, P.loss, P.loss_sum, P.counts};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     P = Predictor{};
@@ -452,17 +554,20 @@ int predictor_setup(Ctx *c, unsigned long long seed, int batch_cap)
         (st = palloc(c, &P.counts, sizeof(int) * 4)))
         return st;
     if (batch_cap > P.batch_cap) {
-        for (void **p : {(void **)&P.X, (void **)&P.Y, (void **)&P.ids, (void **)&P.Z1, (void **)&P.Z2, (void **)&P.z3,
-                         (void **)&P.dZ3, (void **)&P.dZ2, (void **)&P.dZ1, (void **)&P.loss}) {
+        for (void **p : {(void **)&P.X, (void **)&P.Y, (void **)&P.ids, (void **)&P.XT, (void **)&P.H1T, (void **)&P.H2,
+                         (void **)&P.z3, (void **)&P.dZ3, (void **)&P.dZ2, (void **)&P.dZ1, (void **)&P.loss}) {
             if (*p) (void)hipFree(*p);
             *p = nullptr;
         }
         const size_t B = (size_t)batch_cap;
+        P.batch_ld = (batch_cap + 63LL) / 64 * 64;
         if ((st = palloc(c, &P.X, sizeof(float) * NFEAT * B)) || (st = palloc(c, &P.Y, sizeof(float) * B)) ||
-            (st = palloc(c, &P.ids, sizeof(int) * B)) || (st = palloc(c, &P.Z1, sizeof(float) * MLP_H * B)) ||
-            (st = palloc(c, &P.Z2, sizeof(float) * MLP_H * B)) || (st = palloc(c, &P.z3, sizeof(float) * B)) ||
+            (st = palloc(c, &P.ids, sizeof(int) * B)) || (st = palloc(c, &P.XT, sizeof(float) * NFEAT * P.batch_ld)) ||
+            (st = palloc(c, &P.H1T, sizeof(float) * MLP_H * P.batch_ld)) ||
+            (st = palloc(c, &P.H2, sizeof(float) * MLP_H * B)) || (st = palloc(c, &P.z3, sizeof(float) * B)) ||
             (st = palloc(c, &P.dZ3, sizeof(float) * B)) || (st = palloc(c, &P.dZ2, sizeof(float) * MLP_H * B)) ||
-            (st = palloc(c, &P.dZ1, sizeof(float) * MLP_H * B)) || (st = palloc(c, &P.loss, sizeof(float) * B)))
+            (st = palloc(c, &P.dZ1, sizeof(float) * MLP_H * B)) || (st = palloc(c, &P.loss, sizeof(float) * B)) ||
+            (st = palloc(c, &P.loss_sum, sizeof(double))))
             return st;
         P.batch_cap = batch_cap;
     }
@@ -504,11 +609,19 @@ int predictor_get(Ctx *c, int which, float *out)
     return AGAL_OK;
 }
 
+// Wavefronts of the row kernel: one group of rows each, at most four wavefronts per SIMD's worth of
+// workgroups (more rows are looped over, the weights staying in registers).
+static inline unsigned mlp_grid(long long n)
+{
+    const long long per = (PWG / 64) * MLP_R;
+    return (unsigned)std::min<long long>((n + per - 1) / per, 1024);
+}
+
 // Forward on device rows.
-int predictor_forward_dev(Ctx *c, const float *X, int n, float *z3, float *p, float *Z1, float *Z2)
+int predictor_forward_dev(Ctx *c, const float *X, int n, float *z3, float *p)
 {
     if (n <= 0) return AGAL_OK;
-    hipLaunchKernelGGL(k_mlp_forward, dim3(pgrid(n)), dim3(PWG), 0, c->stream, X, n, c->pred.wh, z3, p, Z1, Z2);
+    hipLaunchKernelGGL((k_mlp_rows<false>), dim3(mlp_grid(n)), dim3(PWG), 0, c->stream, X, n, c->pred.wh, z3, p, MlpTrain{});
     AGAL_HIP(c, hipGetLastError());
     return AGAL_OK;
 }
@@ -518,14 +631,10 @@ int predictor_train_dev(Ctx *c, int n, float lr, float pos_weight, double *loss)
 {
     Predictor &P = c->pred;
     if (n <= 0 || n > P.batch_cap) return AGAL_ERR_ARG;
-    int st;
-    if ((st = predictor_forward_dev(c, P.X, n, P.z3, nullptr, P.Z1, P.Z2))) return st;
-    hipLaunchKernelGGL(k_mlp_output_grad, dim3(pgrid(n)), dim3(PWG), 0, c->stream, P.z3, P.Y, n, pos_weight, P.dZ3,
-                       P.loss);
-    hipLaunchKernelGGL(k_mlp_backward, dim3(pgrid(n)), dim3(PWG), 0, c->stream, n, P.wh, P.Z1, P.Z2, P.dZ3, P.dZ2,
-                       P.dZ1);
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3(pgrid(MLP_NPARAM)), dim3(PWG), 0, c->stream, n, P.X, P.Z1, P.Z2, P.dZ3, P.dZ2,
-                       P.dZ1, P.g);
+    const MlpTrain tr{P.Y, pos_weight, P.batch_ld, P.XT, P.H1T, P.H2, P.dZ2, P.dZ1, P.dZ3, P.loss};
+    hipLaunchKernelGGL((k_mlp_rows<true>), dim3(mlp_grid(n)), dim3(PWG), 0, c->stream, P.X, n, P.wh, P.z3, nullptr, tr);
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(WGRAD_WAVES), dim3(64), 0, c->stream, n, P.batch_ld, P.XT, P.H1T, P.H2, P.dZ3,
+                       P.dZ2, P.dZ1, P.loss, P.g, P.loss_sum);
     P.t++;
     const float b1 = 0.9f, b2 = 0.999f;
     const float bc1 = (float)(1.0 - std::pow(0.9, (double)P.t)), bc2 = (float)(1.0 - std::pow(0.999, (double)P.t));
@@ -533,11 +642,9 @@ int predictor_train_dev(Ctx *c, int n, float lr, float pos_weight, double *loss)
                        1e-8f, bc1, bc2);
     AGAL_HIP(c, hipGetLastError());
     if (loss) {
-        std::vector<float> h(n);
-        AGAL_HIP(c, hipMemcpyAsync(h.data(), P.loss, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
-        AGAL_HIP(c, hipStreamSynchronize(c->stream));
         double s = 0;
-        for (float x : h) s += x;
+        AGAL_HIP(c, hipMemcpyAsync(&s, P.loss_sum, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        AGAL_HIP(c, hipStreamSynchronize(c->stream));
         *loss = s / n;
     }
     return AGAL_OK;
@@ -581,7 +688,7 @@ int predictor_features(Ctx *c)
 int predictor_predict_blocks(Ctx *c)
 {
     const int idm = c->id_max[c->MAX_LEVELS];
-    return predictor_forward_dev(c, c->pred.feat, idm, nullptr, c->pred.prob, nullptr, nullptr);
+    return predictor_forward_dev(c, c->pred.feat, idm, nullptr, c->pred.prob);
 }
 
 int predictor_mark(Ctx *c, float thr, int *n_marked)
