@@ -341,45 +341,52 @@ __global__ __launch_bounds__(PWG) void k_mlp_rows(const float *__restrict__ X, i
 }
 
 // Parameter gradients: grad = sum over rows of S[r] V[r][lane], samples summed in order, one
-// wavefront per row of 64 parameters.  The row factor S is the same on every lane (scalar loads
-// from the transposed arrays); 64 rows of V are in flight while the 64 before them are summed, so
-// the wavefront runs near its chain of dependent adds (4096 rows: 1096 us with one thread per
-// parameter and a load per product in the chain).  The last wavefront sums the losses in FP64.
+// wavefront per row of 64 parameters.  The row factors of 64 rows come in one load, a lane each, and
+// go to scalar registers as they are used; 64 rows of V are in flight while the 64 before them are
+// summed, so the wavefront runs near its chain of dependent adds.  4096 rows: 1096 us with one
+// thread per parameter and two loads per link of the chain, 84 us with the factors in scalar loads
+// (each waits for all before it), 49 us so.  The last wavefront sums the losses in FP64.
 constexpr int WG_ROWS = 64;
 
 template <bool HAS_S, bool HAS_V>
 __device__ __forceinline__ float wgrad_sum(int n, const float *__restrict__ S, const float *__restrict__ V, int l)
 {
+    struct Rows {
+        float v[HAS_V ? WG_ROWS : 1], s;
+    };
     float acc = 0.f;
-    float va[WG_ROWS], vb[WG_ROWS];
-    auto load = [&](float *v, int r) {
+    auto load = [&](Rows &R, int r) {
+        if constexpr (HAS_S) R.s = S[r + l];
         if constexpr (HAS_V) {
 #pragma unroll
-            for (int u = 0; u < WG_ROWS; u++) v[u] = V[(long long)(r + u) * MLP_H + l];
+            for (int u = 0; u < WG_ROWS; u++) R.v[u] = V[(long long)(r + u) * MLP_H + l];
         }
     };
-    auto add = [&](const float *v, int r) {
+    auto add = [&](const Rows &R) {
 #pragma unroll
         for (int u = 0; u < WG_ROWS; u++) {
+            float s = 0.f;
+            if constexpr (HAS_S) s = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, R.s), u));
             if constexpr (HAS_S && HAS_V)
-                acc += S[r + u] * v[u];
+                acc += s * R.v[u];
             else if constexpr (HAS_V)
-                acc += v[u];
+                acc += R.v[u];
             else
-                acc += S[r + u];
+                acc += s;
         }
     };
     const int full = n / WG_ROWS * WG_ROWS;
     int r = 0;
-    if (full > 0) load(va, 0);
+    Rows A, B;
+    if (full > 0) load(A, 0);
     for (; r + 2 * WG_ROWS <= full; r += 2 * WG_ROWS) {
-        load(vb, r + WG_ROWS);
-        add(va, r);
-        if (r + 3 * WG_ROWS <= full) load(va, r + 2 * WG_ROWS);
-        add(vb, r + WG_ROWS);
+        load(B, r + WG_ROWS);
+        add(A);
+        if (r + 3 * WG_ROWS <= full) load(A, r + 2 * WG_ROWS);
+        add(B);
     }
     if (r < full) {
-        add(va, r);
+        add(A);
         r += WG_ROWS;
     }
     for (; r < n; r++) {
