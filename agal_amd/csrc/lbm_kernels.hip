@@ -1242,24 +1242,49 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(const int *__restrict__ ids,
 // Coarse -> fine, cubic: Cu_Interpolate_Cubic (solver_lbm_kernels_comm.cu:406-638).  Per parent
 // and direction the 4^d monomial coefficients alpha_i = sum_q C[i][q] s[q] of the tensor-product
 // Lagrange interpolant through the parent's cells are formed once (the reference's coefficient
-// tables, summed term by term in its order), spread over all lanes of the parent's group, and
-// kept in LDS; each child cell then evaluates the polynomial by Horner's rule at its own centre.
-// Same workgroup shape as the linear kernel: one lane per child cell.
+// tables, summed term by term in its order) and kept in LDS; the child cells evaluate the polynomial
+// by Horner's rule in x, then y, then z.
 // ---------------------------------------------------------------------------------------------
 #define AGAL_CUBIC_TABLE __constant__ static const
 #include "cubic_table.inc"
 #undef AGAL_CUBIC_TABLE
 
-constexpr int CWG = 512;  // cubic interpolation: one lane per child cell of a parent
+constexpr int CWG = 512;  // threads of a cubic interpolation workgroup
 
-template <typename T, typename S, int Q, bool ADDED>
-__global__ __launch_bounds__(CWG) void k_interp_cubic(const int *__restrict__ ids, int n, const S *__restrict__ Fp,
-                                                      S *__restrict__ Fc, long long ncm, const int *__restrict__ nbr_child,
-                                                      const int *__restrict__ blk_mask, const int *__restrict__ ref,
-                                                      const int *__restrict__ cells_mask, T tau_ratio)
+// Rescaled populations feq + (f - feq) ratio of one parent cell.
+template <typename T, typename S, int Q>
+__device__ __forceinline__ void rescaled_parent(const S *__restrict__ Fp, long long ncm, long long cell, T ratio, T *s)
 {
     using VS = VelSet<Q>;
-    constexpr int CELLS = VS::CELLS, DIM = VS::DIM, NCH = VS::CHILDREN;
+    T f[Q];
+#pragma unroll
+    for (int p = 0; p < Q; p++) f[p] = Store<T, S>::dec(Fp[(long long)p * ncm + cell], (T)VS::w(p));
+    T rho, u, v, w;
+    moments<T, Q>(f, rho, u, v, w);
+    const T udotu = u * u + v * v + w * w;
+#pragma unroll
+    for (int p = 0; p < Q; p++) {
+        T cdotu = cdot<T, Q>(p, u, v, w);
+        T fe = (T)VS::w(p) * rho * ((T)(1.0) + (T)(3.0) * cdotu + (T)(4.5) * cdotu * cdotu - (T)(1.5) * udotu);
+        s[p] = fe + (f[p] - fe) * ratio;
+    }
+}
+
+// Coordinate of a child cell along one axis in the polynomial's variable: cell 0..7 of the children's
+// row, the second child offset by 2/3.
+template <typename T>
+__device__ __forceinline__ T cubic_coord(int k)
+{
+    const T x = (T)(-0.083333333333333) + (T)(0.166666666666667) * (T)(k & 3);
+    return x + ((k & 4) ? (T)(0.666666666666667) : (T)(0.0));
+}
+
+// 2D: one lane per child cell, eight 4x4 parents per workgroup.
+template <typename T, typename S, int Q, bool ADDED>
+__device__ __forceinline__ void interp_cubic_2d(const InterpArgs<T, S> &ia)
+{
+    using VS = VelSet<Q>;
+    constexpr int CELLS = VS::CELLS, NCH = VS::CHILDREN;
     constexpr int GROUP = NCH * CELLS;
     constexpr int PPW = CWG / GROUP;
     __shared__ T s_all[Q * PPW * CELLS];  // rescaled parent populations, [p][parent][cell]
@@ -1268,72 +1293,154 @@ __global__ __launch_bounds__(CWG) void k_interp_cubic(const int *__restrict__ id
     const int c = r / CELLS, t = r % CELLS;
     const int bi = blockIdx.x * PPW + g;
     int b = -1;
-    if (bi < n) b = ids[bi];
+    if (bi < ia.n) b = ia.ids[bi];
     bool work = false;
     int fc = 0;
     if (b >= 0) {
-        fc = nbr_child[b];
-        work = fc >= 0 && (ADDED ? (ref[b] == REF_MARK_REFINE) : (blk_mask[b] == BLK_INTERFACE));
+        fc = ia.nbr_child[b];
+        work = fc >= 0 && (ADDED ? (ia.ref[b] == REF_MARK_REFINE) : (ia.blk_mask[b] == BLK_INTERFACE));
     }
     if (work && c == 0) {
-        const long long cell = (long long)b * CELLS + t;
-        T f[Q];
+        T s[Q];
+        rescaled_parent<T, S, Q>(ia.Fp, ia.ncm, (long long)b * CELLS + t, ia.tau_ratio, s);
 #pragma unroll
-        for (int p = 0; p < Q; p++) f[p] = Store<T, S>::dec(Fp[(long long)p * ncm + cell], (T)VS::w(p));
-        T rho, u, v, w;
-        moments<T, Q>(f, rho, u, v, w);
-        const T udotu = u * u + v * v + w * w;
-#pragma unroll
-        for (int p = 0; p < Q; p++) {
-            T cdotu = cdot<T, Q>(p, u, v, w);
-            T fe = (T)VS::w(p) * rho * ((T)(1.0) + (T)(3.0) * cdotu + (T)(4.5) * cdotu * cdotu - (T)(1.5) * udotu);
-            s_all[(p * PPW + g) * CELLS + t] = fe + (f[p] - fe) * tau_ratio;
-        }
+        for (int p = 0; p < Q; p++) s_all[(p * PPW + g) * CELLS + t] = s[p];
     }
     __syncthreads();
     if (work) {
-        const int *start = (DIM == 3) ? CUBIC3_START : CUBIC2_START;
-        const unsigned char *qs = (DIM == 3) ? CUBIC3_Q : CUBIC2_Q;
-        const double *cs = (DIM == 3) ? CUBIC3_C : CUBIC2_C;
         for (int k = r; k < Q * CELLS; k += GROUP) {
             const int p = k / CELLS, i = k % CELLS;
             const T *s = s_all + (p * PPW + g) * CELLS;
-            T acc = (T)cs[start[i]] * s[qs[start[i]]];
-            for (int m = start[i] + 1; m < start[i + 1]; m++) acc = acc + (T)cs[m] * s[qs[m]];
+            T acc = (T)CUBIC2_C[CUBIC2_START[i]] * s[CUBIC2_Q[CUBIC2_START[i]]];
+            for (int m = CUBIC2_START[i] + 1; m < CUBIC2_START[i + 1]; m++) acc = acc + (T)CUBIC2_C[m] * s[CUBIC2_Q[m]];
             a_all[(p * PPW + g) * CELLS + i] = acc;
         }
     }
     __syncthreads();
     if (!work) return;
     const long long ccell = (long long)(fc + c) * CELLS + t;
-    if (!ADDED && cells_mask[ccell] != CELL_GHOST) return;
-    const T M_ONE_TWELFTH = (T)(-0.083333333333333), ONE_SIXTH = (T)(0.166666666666667);
-    const T TWO_THIRDS = (T)(0.666666666666667), ZERO_THIRDS = (T)(0.0);
-    const int I = t % 4, J = (t / 4) % 4, K = (DIM == 3) ? t / 16 : 0;
-    const T x = M_ONE_TWELFTH + ONE_SIXTH * (T)I;
-    const T y = M_ONE_TWELFTH + ONE_SIXTH * (T)J;
-    const T z = (DIM == 3) ? M_ONE_TWELFTH + ONE_SIXTH * (T)K : (T)0;
-    const T ox = (c & 1) ? TWO_THIRDS : ZERO_THIRDS, oy = (c & 2) ? TWO_THIRDS : ZERO_THIRDS;
-    const T oz = (c & 4) ? TWO_THIRDS : ZERO_THIRDS;
+    if (!ADDED && ia.cells_mask[ccell] != CELL_GHOST) return;
+    const T x = cubic_coord<T>((t & 3) + 4 * (c & 1)), y = cubic_coord<T>((t >> 2) + 4 * (c >> 1));
 #pragma unroll 1
     for (int p = 0; p < Q; p++) {
         const T *al = a_all + (p * PPW + g) * CELLS;
         T res = 0;
 #pragma unroll
-        for (int mk = 0; mk < (DIM == 3 ? 4 : 1); mk++) {
-            T gam = 0;
+        for (int mj = 0; mj < 4; mj++) {
+            T beta = 0;
+#pragma unroll
+            for (int mi = 0; mi < 4; mi++) beta = al[(3 - mi) + 4 * (3 - mj)] + x * beta;
+            res = beta + y * res;
+        }
+        ia.Fc[(long long)p * ia.ncm + ccell] = Store<T, S>::enc(res, (T)VS::w(p));
+    }
+}
+
+// 3D: one workgroup of eight wavefronts per parent.  The coefficients: lane (p, g) of a wavefront
+// forms alpha_i of direction p for one of G = 64 / Q indices i at a time, the indices dealt out by
+// falling number of terms (64, 16, 4 or 1), so a wavefront's lanes run chains of equal length and
+// their LDS reads s[q][p] fall in consecutive banks.  The values: a wavefront takes one direction,
+// lane (x, y) of the children's 8 x 8 columns forms the four z-coefficients once (Horner in x, then
+// y) and runs down the eight z: 14 multiply-adds per child cell instead of 84, each the same
+// operation on the same operands.  FP64 vector issue and LDS latency bound it.  Three levels on a
+// 32^3 root in FP64 (launches of 176 and 736 parents): 28.8 us a launch, 130 us with one lane per
+// child cell.
+struct CubicOrder {
+    unsigned char i[64];
+};
+constexpr CubicOrder make_cubic_order()
+{
+    CubicOrder o{};
+    int n = 0;
+    for (int nz = 3; nz >= 0; nz--)  // an index has 4 terms for every nonzero digit (power of x, y, z)
+        for (int i = 0; i < 64; i++)
+            if ((i % 4 != 0) + (i / 4 % 4 != 0) + (i / 16 != 0) == nz) o.i[n++] = (unsigned char)i;
+    return o;
+}
+__constant__ const CubicOrder kCubicOrder = make_cubic_order();
+
+template <typename T, typename S, int Q, bool ADDED>
+__device__ __forceinline__ void interp_cubic_3d(const InterpArgs<T, S> &ia)
+{
+    using VS = VelSet<Q>;
+    constexpr int NW = CWG / 64, G = 64 / Q, AL = 66;
+    __shared__ T s_par[64 * Q];   // rescaled parent populations, [cell][p]
+    __shared__ __attribute__((aligned(16))) T s_al[Q * AL];  // monomial coefficients, [p][i]
+    const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int b = ia.ids[blockIdx.x];
+    const int fc = ia.nbr_child[b];
+    // The same for the whole workgroup.
+    if (fc < 0 || !(ADDED ? (ia.ref[b] == REF_MARK_REFINE) : (ia.blk_mask[b] == BLK_INTERFACE))) return;
+    if (wv == 0) {
+        T s[Q];
+        rescaled_parent<T, S, Q>(ia.Fp, ia.ncm, (long long)b * 64 + l, ia.tau_ratio, s);
+#pragma unroll
+        for (int p = 0; p < Q; p++) s_par[l * Q + p] = s[p];
+    }
+    // This lane's column of child cells, and which of them are written (bit z).
+    const int cx = l & 7, cy = l >> 3;
+    const long long col = (long long)(fc + (cx >> 2) + 2 * (cy >> 2)) * 64 + (cx & 3) + 4 * (cy & 3);
+    unsigned put = 0xffu;
+    if (!ADDED) {
+        put = 0;
+#pragma unroll
+        for (int z = 0; z < 8; z++)
+            put |= (ia.cells_mask[col + (z >> 2) * 256 + (z & 3) * 16] == CELL_GHOST ? 1u : 0u) << z;
+    }
+    __syncthreads();
+    const int p1 = l % Q, g = l / Q;
+    for (int k = wv; k < (64 + G - 1) / G; k += NW) {
+        const int at = k * G + g;
+        if (g >= G || at >= 64) continue;
+        const int i = kCubicOrder.i[at], m0 = CUBIC3_START[i], m1 = CUBIC3_START[i + 1];
+        const T *s = s_par + p1;
+        T acc = (T)CUBIC3_C[m0] * s[CUBIC3_Q[m0] * Q];
+#pragma unroll 8
+        for (int m = m0 + 1; m < m1; m++) acc = acc + (T)CUBIC3_C[m] * s[CUBIC3_Q[m] * Q];
+        s_al[p1 * AL + i] = acc;
+    }
+    __syncthreads();
+    const T x = cubic_coord<T>(cx), y = cubic_coord<T>(cy);
+#pragma unroll 1
+    for (int p = wv; p < Q; p += NW) {
+        const T *al = s_al + p * AL;
+        T gam[4];
+#pragma unroll
+        for (int mk = 0; mk < 4; mk++) {
+            T gm = 0;
 #pragma unroll
             for (int mj = 0; mj < 4; mj++) {
                 T beta = 0;
 #pragma unroll
-                for (int mi = 0; mi < 4; mi++)
-                    beta = al[(3 - mi) + 4 * (3 - mj) + (DIM == 3 ? 16 * (3 - mk) : 0)] + (x + ox) * beta;
-                gam = beta + (y + oy) * gam;
+                for (int mi = 0; mi < 4; mi++) beta = al[(3 - mi) + 4 * (3 - mj) + 16 * (3 - mk)] + x * beta;
+                gm = beta + y * gm;
             }
-            res = (DIM == 3) ? gam + (z + oz) * res : gam;
+            gam[mk] = gm;
         }
-        Fc[(long long)p * ncm + ccell] = Store<T, S>::enc(res, (T)VS::w(p));
+        // The direction is the same on the whole wavefront: a constant weight per branch.
+        T wp = 0;
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (q == p) wp = (T)VS::w(q);
+        S *row = ia.Fc + (long long)p * ia.ncm + col;
+#pragma unroll
+        for (int z = 0; z < 8; z++) {
+            const T zz = cubic_coord<T>(z);
+            T res = 0;
+#pragma unroll
+            for (int mk = 0; mk < 4; mk++) res = gam[mk] + zz * res;
+            if ((put >> z) & 1) row[(z >> 2) * 256 + (z & 3) * 16] = Store<T, S>::enc(res, wp);
+        }
     }
+}
+
+template <typename T, typename S, int Q, bool ADDED>
+__global__ __launch_bounds__(CWG) void k_interp_cubic(InterpArgs<T, S> ia)
+{
+    if constexpr (VelSet<Q>::DIM == 3)
+        interp_cubic_3d<T, S, Q, ADDED>(ia);
+    else
+        interp_cubic_2d<T, S, Q, ADDED>(ia);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1919,7 +2026,7 @@ static inline int interp_grid(long long nparents)
 template <int Q>
 static inline int cubic_grid(long long nparents)
 {
-    constexpr int ppw = CWG / (VelSet<Q>::CHILDREN * VelSet<Q>::CELLS);
+    constexpr int ppw = VelSet<Q>::DIM == 3 ? 1 : CWG / (VelSet<Q>::CHILDREN * VelSet<Q>::CELLS);
     return (int)((nparents + ppw - 1) / ppw);
 }
 
@@ -2291,13 +2398,11 @@ static int interpolate_t(Ctx *c, int L, int var)
     hipStream_t s = sched_begin(c, 0, rl, wl);
     if (c->P.interp_order == AGAL_INTERP_CUBIC) {
         if (var == AGAL_INTERP_ADDED)
-            hipLaunchKernelGGL((k_interp_cubic<T, S, Q, true>), dim3(cubic_grid<Q>(n)), dim3(CWG), 0, s, ids, n,
-                               Fbuf<S>(c, c->cur[L]), Fbuf<S>(c, c->cur[L + 1]), c->n_maxcells, c->nbr_child,
-                               c->blk_mask, c->ref, c->cells_mask, ratio);
+            hipLaunchKernelGGL((k_interp_cubic<T, S, Q, true>), dim3(cubic_grid<Q>(n)), dim3(CWG), 0, s,
+                               interp_args<T, S>(c, L, ids, n, ratio));
         else
-            hipLaunchKernelGGL((k_interp_cubic<T, S, Q, false>), dim3(cubic_grid<Q>(n)), dim3(CWG), 0, s, ids, n,
-                               Fbuf<S>(c, c->cur[L]), Fbuf<S>(c, c->cur[L + 1]), c->n_maxcells, c->nbr_child,
-                               c->blk_mask, c->ref, c->cells_mask, ratio);
+            hipLaunchKernelGGL((k_interp_cubic<T, S, Q, false>), dim3(cubic_grid<Q>(n)), dim3(CWG), 0, s,
+                               interp_args<T, S>(c, L, ids, n, ratio));
     } else if (var == AGAL_INTERP_ADDED)
         hipLaunchKernelGGL((k_interp<T, S, Q, true>), dim3(interp_grid<Q>(n)), dim3(IWG), 0, s,
                            interp_args<T, S>(c, L, ids, n, ratio));

@@ -7,8 +7,8 @@ import pytest
 
 from agal_amd import capi
 from agal_amd.mesh import LbmMesh
-from oracle_lib import MlpOracle
-from parity import ldc_params
+from oracle_lib import MlpOracle, OracleMesh
+from parity import compare_states, ldc_params
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +32,18 @@ def test_forward_and_gradients_at_the_edges_of_row_groups(n):
     assert abs(lg - lo) <= 1e-5 * max(1.0, abs(lo))
     np.testing.assert_allclose(g.predictor_params(2), o.g, rtol=0, atol=max(1e-6, n * 2.0 ** -24) * np.abs(o.g).max())
     g.close()
+
+
+@pytest.mark.parametrize("vs,prec", [(capi.D3Q27, capi.FP16), (capi.D3Q27, capi.FP64), (capi.D3Q19, capi.BF16)])
+def test_cubic_interpolation_of_other_sets_and_storage(vs, prec):
+    """The cubic kernel's lanes are dealt by the number of directions (two index groups for 27, three
+    for 19): interface and new children of three levels, bit for bit."""
+    p = ldc_params(vs=vs, N=16, Re=40.0, levels=3, P_REFINE=8, prec=prec, interp_order=capi.INTERP_CUBIC,
+                   N_REFINE_START=-2)
+    g, o = LbmMesh(p, 8192), OracleMesh(p, 8192)
+    for m in (g, o):
+        m.S_SetIC(0)
+        m.advance_loop(0, 24)
+    assert g.refresh_sizes().n_ids[1] > 0
+    bad = compare_states(g.state(), o.state())
+    assert not bad, "\n".join(bad)
