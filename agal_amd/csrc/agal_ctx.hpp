@@ -77,6 +77,7 @@ struct Ctx {
 
     // Host mirrors of the pool bookkeeping (inc/mesh.h:447-462).
     std::vector<int> n_ids, id_max, n_iface;
+    std::vector<int> n_general;  // blocks per level that are not simple, or whose neighbour slots are not mutual
     int n_gaps = 0;
     std::vector<int> cur;  // current population buffer per level
     int global_Liter = 0;
@@ -98,14 +99,16 @@ struct Ctx {
     int *first_child = nullptr, *scan_a = nullptr, *scan_b = nullptr, *partials = nullptr;
     int *dscal = nullptr;     // small device scalars (counters)
     int *hscal = nullptr;     // pinned host mirror
-    // Exceptions of the stream guard: (initiator cell, partner cell, direction) + value, one list
-    // of exc_cap entries per level.
+    // Exceptions of the stream guard: (initiator cell, partner cell, direction) + value, lists of
+    // exc_cap entries: 2L and 2L + 1 of level L, used in turn, and the extra list 2 MAX_LEVELS.
     long long exc_cap = 0, exc_cap_alloc = 0;
     bool exc_overflowed = false;  // an overflow was reported: steps are refused
     int *exc_idx = nullptr;   // 3 ints per entry
     void *exc_val = nullptr;  // one value per entry
-    int *exc_count = nullptr; // per level (and the extra slot MAX_LEVELS): [2L] count, [2L+1] overflow flag
-    // The extra list (slot MAX_LEVELS) linked per block: chain heads per block ID (-1 when empty)
+    // Per list k: [2k] count, [2k+1] overflow flag; then the seven hand-over counters of the kernels
+    // that resolve pending lists.
+    int *exc_count = nullptr;
+    // The extra list linked per block: chain heads per block ID (-1 when empty)
     // and two links per entry (through its initiator's and its partner's block).
     int *exc_head = nullptr, *exc_next = nullptr;
 
@@ -172,9 +175,23 @@ struct Ctx {
     // read).  Only while a coarse step is being issued (defer_coarse).
     bool defer_coarse = false;
     std::vector<std::pair<int, int>> deferred;
-    // Exception lists awaiting their fixup: (level, buffer the level's launch wrote).  Resolved
-    // before anything else touches the level, or by workgroups of a fused launch that does not.
-    std::vector<std::pair<int, int>> pending_fix;
+    // Exception lists awaiting their fixup: level, buffer the level's launch wrote, and whether the list
+    // is that of an in-place pair's first sub-step.  Resolved by the next kernel that can (it waits for
+    // it before it starts), or by a launch of its own.
+    struct PendingFix {
+        int L, buf, exchange, slot;
+    };
+    std::vector<PendingFix> pending_fix;
+    int exc_turn[8] = {};  // which of its two lists a level records into next
+    int exc_slot(int L) const { return 2 * L + exc_turn[L]; }
+    int exc_extra() const { return 2 * MAX_LEVELS; }
+    int exc_lists() const { return 2 * MAX_LEVELS + 1; }
+    // The list that a launch of level L has recorded into (buffer buf) awaits its fixup.
+    void leave_pending(int L, int buf, int exchange)
+    {
+        pending_fix.push_back({L, buf, exchange, exc_slot(L)});
+        exc_turn[L] ^= 1;
+    }
     // 1 while the first, 2 while the second sub-step of a finest-level pair is issued, else 0.
     int fine_pair = 0;
     hipStream_t lstream[8] = {};
@@ -210,8 +227,10 @@ int launch_set_ic(Ctx *c, int L);
 int launch_refresh(Ctx *c, int L);
 int launch_collide_stream(Ctx *c, int L);
 int launch_flush_deferred(Ctx *c);
+// The second sub-step of an in-place pair (lbm_inplace.hip).
+int launch_odd_step(Ctx *c, int L);
+bool inplace_pair(const Ctx *c, int L);
 int launch_interp_collide(Ctx *c, int L);
-int launch_fix_pending(Ctx *c);
 int launch_interpolate(Ctx *c, int L, int var);
 int launch_average(Ctx *c, int L, int var);
 // average(L) in the advance's mode followed by interpolate(L, INTERFACE), fused for linear

@@ -488,23 +488,28 @@ __global__ void k_block_aux(const int *nbr, const int *nbr_child, const int *blk
 // step then skips the guard reads).  2: in addition every neighbour slot that the velocity set
 // links to exists (so no link leaves the domain or the level) and slot 13 is the block itself --
 // the fused step's interior path.  max_nz: most nonzero components of a link (2 for D3Q19).
+// n_general[L] counts the active blocks of level L that are not simple, or have a neighbour that is not
+// of their level or does not have them in its opposite slot: the levels without one may step in place.
 template <int DIM>
-__global__ void k_block_simple(const int *nbr_slot, const int *part, const int *has_solid, int *simple, int n,
-                               int max_nz)
+__global__ void k_block_simple(const int *nbr_slot, const int *part, const int *has_solid, const int *ref,
+                               const int *level, int *simple, int n, int max_nz, int *n_general)
 {
     constexpr int QMAX = DIM == 3 ? 27 : 9;
     int kap = blockIdx.x * AWG + threadIdx.x;
     if (kap >= n) return;
     int s = part[kap] && !has_solid[kap];
-    bool all = true;
+    bool all = true, mutual = true;
     for (int S = 0; S < QMAX && s; S++) {
         int nb = nbr_slot[(long long)kap * QMAX + S];
         if (nb >= 0 && (!part[nb] || has_solid[nb])) s = 0;
+        if (nb >= 0 && (nbr_slot[(long long)nb * QMAX + QMAX - 1 - S] != kap || level[nb] != level[kap])) mutual = false;
         const int nz = (S % 3 != 1) + ((S / 3) % 3 != 1) + (DIM == 3 ? (S / 9 != 1) : 0);
         if (nb < 0 && nz <= max_nz) all = false;
     }
     if (s && all && nbr_slot[(long long)kap * QMAX + (QMAX - 1) / 2] == kap) s = 2;
     simple[kap] = s;
+    // Slot 13 (4 in 2D) is its own opposite: mutual only if it is the block itself.
+    if ((s == 0 || !mutual) && ref[kap] != REF_INACTIVE) atomicAdd(&n_general[level[kap]], 1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -739,7 +744,6 @@ static int build_traversal_order(Ctx *c)
     if (c->n_ids[0] > 0)
         AGAL_HIP(c, hipMemcpyAsync(c->order_L(0), c->id_set_L(0), sizeof(int) * c->n_ids[0], hipMemcpyDeviceToDevice,
                                    c->stream));
-    if ((st = launch_fill(c, c->dscal + 16, 16, 0))) return st;
     for (int L = 1; L < ML; L++) {
         st = compact(c, PredActiveChildren{c->order_L(L - 1), c->nbr_child, c->ref, c->level, L}, c->n_ids[L - 1],
                      EmitChildren{c->order_L(L - 1), c->nbr_child, c->order_L(L), c->NCH}, c->dscal + 16 + L);
@@ -747,6 +751,7 @@ static int build_traversal_order(Ctx *c)
     }
     AGAL_HIP(c, hipMemcpyAsync(c->hscal + 16, c->dscal + 16, sizeof(int) * 16, hipMemcpyDeviceToHost, c->stream));
     AGAL_HIP(c, hipStreamSynchronize(c->stream));
+    for (int L = 0; L < ML; L++) c->n_general[L] = c->hscal[24 + L];
     for (int L = 1; L < ML; L++)
         if ((long long)c->hscal[16 + L] * c->NCH != c->n_ids[L] && c->n_ids[L] > 0)
             AGAL_HIP(c, hipMemcpyAsync(c->order_L(L), c->id_set_L(L), sizeof(int) * c->n_ids[L], hipMemcpyDeviceToDevice,
@@ -780,23 +785,26 @@ int rebuild_level_lists(Ctx *c, long long range_hint)
             AGAL_HIP(c, hipMemcpyAsync(&last[L], c->id_set_L(L) + c->n_ids[L] - 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     if ((st = read_scalars(c, 16))) return st;
     for (int L = 0; L < ML; L++) c->n_iface[L] = c->hscal[8 + L];
-    if ((st = build_traversal_order(c))) return st;
-    c->mesh_epoch++;  // recorded step graphs carry the old list sizes
     for (int L = 1; L < ML; L++) c->id_max[L] = c->n_ids[L] > 0 ? last[L] + 1 : 0;
     c->id_max[ML] = *std::max_element(c->id_max.begin(), c->id_max.begin() + ML);
-    int n = c->id_max[ML];
+    // Block flags; dscal[24..24+ML): per-level counts of blocks that cannot step in place, read with the
+    // traversal's counts.
+    if ((st = launch_fill(c, c->dscal + 16, 16, 0))) return st;
+    const int n = c->id_max[ML];
     if (c->DIM == 3) {
         hipLaunchKernelGGL((k_block_aux<3>), dim3(grid1(n)), dim3(AWG), 0, c->stream, c->nbr, c->nbr_child, c->blk_mask,
                            c->cells_mask, c->nbr_slot, c->part, c->scan_a, c->n_maxcblocks, n);
         hipLaunchKernelGGL((k_block_simple<3>), dim3(grid1(n)), dim3(AWG), 0, c->stream, c->nbr_slot, c->part, c->scan_a,
-                           c->simple, n, c->Q == 27 ? 3 : 2);
+                           c->ref, c->level, c->simple, n, c->Q == 27 ? 3 : 2, c->dscal + 24);
     } else {
         hipLaunchKernelGGL((k_block_aux<2>), dim3(grid1(n)), dim3(AWG), 0, c->stream, c->nbr, c->nbr_child, c->blk_mask,
                            c->cells_mask, c->nbr_slot, c->part, c->scan_a, c->n_maxcblocks, n);
         hipLaunchKernelGGL((k_block_simple<2>), dim3(grid1(n)), dim3(AWG), 0, c->stream, c->nbr_slot, c->part, c->scan_a,
-                           c->simple, n, 2);
+                           c->ref, c->level, c->simple, n, 2, c->dscal + 24);
     }
     AGAL_HIP(c, hipGetLastError());
+    if ((st = build_traversal_order(c))) return st;
+    c->mesh_epoch++;  // recorded step graphs carry the old list sizes
     // The linked blocks of the new level lists (their ranks and fractions stay with the block IDs).
     return links_rebuild_lists(c);
 }

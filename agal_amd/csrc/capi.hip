@@ -308,7 +308,6 @@ int advance_rec(Ctx *c, int L)
             c->global_Liter = 0;
             if ((st = launch_interp_collide(c, L))) return st;
             if ((st = advance_rec(c, L + 1))) return st;
-            if ((st = launch_fix_pending(c))) return st;
             if ((st = launch_average(c, L, average_advance(c)))) return st;
         } else {
             if (L < ML - 1) {
@@ -324,7 +323,6 @@ int advance_rec(Ctx *c, int L)
             if (L == ML - 1) c->global_Liter++;
             if (L < ML - 1) {
                 if ((st = advance_rec(c, L + 1))) return st;
-                if ((st = launch_fix_pending(c))) return st;
                 if ((st = launch_average_interpolate(c, L))) return st;
             }
             if (L == ML - 1) c->fine_pair = 2;
@@ -334,7 +332,6 @@ int advance_rec(Ctx *c, int L)
             if (L == ML - 1) c->global_Liter++;
             if (L < ML - 1) {
                 if ((st = advance_rec(c, L + 1))) return st;
-                if ((st = launch_fix_pending(c))) return st;
                 if ((st = launch_average(c, L, average_advance(c)))) return st;
             }
         }
@@ -379,6 +376,36 @@ int advance_step(Ctx *c, int L0)
     return launch_mea_post(c);
 }
 
+// `k` consecutive coarse steps from level L0.  Without refinement the steps have nothing between them:
+// each resolves the exception list of the one before as it starts, and two at a time run as in-place
+// pairs where the level allows it.
+int advance_steps(Ctx *c, int L0, int k)
+{
+    int st = AGAL_OK;
+    const bool multi = c->MAX_LEVELS > 1 && c->MAX_LEVELS != L0 + 1;
+    if (!multi && !c->cv_F && !c->links_on) {
+        const bool pairs = inplace_pair(c, L0);
+        c->defer_coarse = true;
+        while (k > 0 && st == AGAL_OK) {
+            c->fine_pair = pairs && k >= 2 ? 1 : 0;
+            st = launch_collide_stream(c, L0);
+            if (c->fine_pair && st == AGAL_OK) {
+                c->fine_pair = 2;
+                st = launch_collide_stream(c, L0);
+                k--;
+            }
+            k--;
+        }
+        c->fine_pair = 0;
+        c->defer_coarse = false;
+        const int st2 = launch_flush_deferred(c);
+        return st ? st : st2;
+    }
+    for (; k > 0; k--)
+        if ((st = advance_step(c, L0))) return st;
+    return AGAL_OK;
+}
+
 unsigned cur_mask(const Ctx *c)
 {
     unsigned m = 0;
@@ -400,9 +427,7 @@ int steps_once(Ctx *c, int L0, int k)
 {
     int st;
     if (!c->use_graphs || c->timing.enabled || L0 != c->N_LEVEL_START) {
-        for (int j = 0; j < k; j++)
-            if ((st = advance_step(c, L0))) return st;
-        return AGAL_OK;
+        return advance_steps(c, L0, k);
     }
     const unsigned before = cur_mask(c);
     for (auto &g : c->graphs)
@@ -440,7 +465,7 @@ int steps_once(Ctx *c, int L0, int k)
     hipError_t e = hipEventRecord(c->sched_start, c->stream);
     if (e != hipSuccess) st = hip_fail(c, e, "hipEventRecord");
     c->sched_on = (st == AGAL_OK);
-    for (int j = 0; j < k && st == AGAL_OK; j++) st = advance_step(c, L0);
+    if (st == AGAL_OK) st = advance_steps(c, L0, k);
     c->sched_on = false;
     for (int k = 1; k < Ctx::NSLOT; k++) {  // joined also after a failure so that the capture can end
         if (!c->slot_joined[k]) continue;
@@ -699,12 +724,12 @@ int refine_near_wall_impl(Ctx *c)
 int check_exceptions(Ctx *c)
 {
     if (c->exc_overflowed) return AGAL_ERR_OVERFLOW;
-    std::vector<int> v(2 * (c->MAX_LEVELS + 1), 0);
+    std::vector<int> v(2 * c->exc_lists(), 0);
     AGAL_HIP(c, hipMemcpyAsync(v.data(), c->exc_count, sizeof(int) * v.size(), hipMemcpyDeviceToHost, c->stream));
     AGAL_HIP(c, hipStreamSynchronize(c->stream));
-    for (int L = 0; L <= c->MAX_LEVELS; L++)
-        if (v[2 * L + 1]) {
-            c->last_error = "stream-guard exception list of level " + std::to_string(L) + " overflowed (" +
+    for (int k = 0; k < c->exc_lists(); k++)
+        if (v[2 * k + 1]) {
+            c->last_error = "stream-guard exception list of level " + std::to_string(std::min(k / 2, c->MAX_LEVELS - 1)) + " overflowed (" +
                             std::to_string(c->exc_cap) + " entries): populations are invalid, the context refuses "
                             "further steps";
             c->exc_overflowed = true;
@@ -887,6 +912,7 @@ int agal_create(const agal_params *p, long long block_capacity, int device, agal
         compute_level_params<float>(c);
     c->n_ids.assign(c->MAX_LEVELS + 1, 0);
     c->n_iface.assign(c->MAX_LEVELS + 1, 0);
+    c->n_general.assign(c->MAX_LEVELS + 1, 0);
     c->id_max.assign(c->MAX_LEVELS + 1, 0);
     c->cur.assign(c->MAX_LEVELS, 0);
 
@@ -942,11 +968,11 @@ int agal_create(const agal_params *p, long long block_capacity, int device, agal
     ALLOC(c->scan_b, sizeof(int) * nmax);
     ALLOC(c->partials, sizeof(int) * ((nmax + 2047) / 2048 + 64));
     ALLOC(c->dscal, sizeof(int) * 64);
-    // One exception list per level, and one more (slot MAX_LEVELS) that the first sub-step of each
-    // finest-level pair writes for the second to apply as it loads.
-    ALLOC(c->exc_idx, sizeof(int) * 3 * c->exc_cap * (c->MAX_LEVELS + 1));
-    ALLOC(c->exc_val, cs * c->exc_cap * (c->MAX_LEVELS + 1));
-    ALLOC(c->exc_count, sizeof(int) * 2 * (c->MAX_LEVELS + 1));
+    // Two exception lists per level, and one more that the first sub-step of a finest-level pair that is
+    // not in place writes for the second to apply as it loads.
+    ALLOC(c->exc_idx, sizeof(int) * 3 * c->exc_cap * c->exc_lists());
+    ALLOC(c->exc_val, cs * c->exc_cap * c->exc_lists());
+    ALLOC(c->exc_count, sizeof(int) * (2 * c->exc_lists() + 7));
     ALLOC(c->exc_head, sizeof(int) * nmax);
     ALLOC(c->exc_next, sizeof(int) * 2 * c->exc_cap_alloc);
     if (c->P.S_FORCE_TYPE == 1) ALLOC(c->cv_F, cs * 6 * nmax);
@@ -963,7 +989,7 @@ int agal_create(const agal_params *p, long long block_capacity, int device, agal
     if ((st = fill(c->cells_mask, ncm, CELL_INTERIOR)) || (st = fill(c->blk_mask, nmax, BLK_REGULAR)) ||
         (st = fill(c->nbr, c->QMAX * nmax, N_SKIPID)) || (st = fill(c->nbr_child, c->QMAX * nmax, N_SKIPID)) ||
         (st = fill(c->ref, nmax, REF_INACTIVE)) || (st = fill(c->level, nmax, 0)) || (st = fill(c->onb, nmax, 0)) ||
-        (st = fill((int *)c->map_stamp, nmax, 0)) || (st = fill(c->exc_count, 2 * (c->MAX_LEVELS + 1), 0)) || (st = fill(c->exc_head, nmax, -1)) || (st = fill(c->part, nmax, 1)) ||
+        (st = fill((int *)c->map_stamp, nmax, 0)) || (st = fill(c->exc_count, 2 * c->exc_lists() + 7, 0)) || (st = fill(c->exc_head, nmax, -1)) || (st = fill(c->part, nmax, 1)) ||
         (st = fill(c->simple, nmax, 0)) || (st = fill((int *)c->X, c->DIM * nmax, 0)) ||
         (c->cv_F && (st = fill((int *)c->cv_F, (long long)(cs / 4) * 6 * nmax, 0)))) {
         free_ctx(c);
@@ -1673,7 +1699,7 @@ int agal_import_pool(agal_ctx *ctx, const agal_pool *pl)
     std::fill(c->cur.begin(), c->cur.end(), 0);
     c->pending_fix.clear();
     c->deferred.clear();
-    if ((st = launch_fill(c, c->exc_count, 2 * (ML + 1), 0))) return st;
+    if ((st = launch_fill(c, c->exc_count, 2 * c->exc_lists() + 7, 0))) return st;
     if ((st = rebuild_level_lists(c, nb))) return st;
     if (pl->populations) {
         c->ic_done = true;

@@ -21,69 +21,9 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-
-#include "agal_common.hpp"
-#include "agal_ctx.hpp"
+#include "lbm_device.hpp"
 
 namespace agal {
-
-constexpr int WG = 256;
-
-// Moments in the reference's order (p-order sums, then division): Cu_RefreshVariables (:110-159).
-// The reference adds c * f for every component, zeros included; those terms are left out here.
-// A sum that starts at +0 never becomes -0 under round-to-nearest, so adding 0 * f = +-0 leaves
-// it unchanged: for finite populations the results are the same bits, at about a third fewer
-// vector instructions.
-template <typename T, int Q>
-__device__ __forceinline__ void moments(const T *f, T &rho, T &u, T &v, T &w)
-{
-    using VS = VelSet<Q>;
-    rho = 0;
-    u = 0;
-    v = 0;
-    w = 0;
-#pragma unroll
-    for (int p = 0; p < Q; p++) {
-        rho += f[p];
-        if (VS::cx(p) > 0) u += f[p];
-        if (VS::cx(p) < 0) u -= f[p];
-        if (VS::cy(p) > 0) v += f[p];
-        if (VS::cy(p) < 0) v -= f[p];
-        if (VS::DIM == 3 && VS::cz(p) > 0) w += f[p];
-        if (VS::DIM == 3 && VS::cz(p) < 0) w -= f[p];
-    }
-    // One correctly rounded division, then products (the CPU restatement does the same).
-    const T r = (T)(1.0) / rho;
-    u = u * r;
-    v = v * r;
-    if (VS::DIM == 3) w = w * r;
-}
-
-// c_p . u in the reference's left-to-right order (cx u + cy v) + cz w, without the terms of zero
-// components.  A nonzero sum is unchanged by them; a zero sum may differ in sign only, which the
-// equilibrium polynomial 1 + 3 c.u + 4.5 (c.u)^2 does not see.
-template <typename T, int Q>
-__device__ __forceinline__ T cdot(int p, T u, T v, T w)
-{
-    using VS = VelSet<Q>;
-    T s = (T)0;
-    bool first = true;
-    if (VS::cx(p) != 0) {
-        s = VS::cx(p) > 0 ? u : -u;
-        first = false;
-    }
-    if (VS::cy(p) != 0) {
-        const T t = VS::cy(p) > 0 ? v : -v;
-        s = first ? t : s + t;
-        first = false;
-    }
-    if (VS::DIM == 3 && VS::cz(p) != 0) {
-        const T t = VS::cz(p) > 0 ? w : -w;
-        s = first ? t : s + t;
-    }
-    return s;
-}
 
 // ---------------------------------------------------------------------------------------------
 // Initial conditions: Cu_SetInitialConditions (solver_lbm_kernels.cu:13-77), uniform state hook.
@@ -129,790 +69,6 @@ __global__ __launch_bounds__(WG) void k_refresh(const int *__restrict__ ids, int
     M[1 * ncm + cell] = u;
     M[2 * ncm + cell] = v;
     M[3 * ncm + cell] = (VS::DIM == 3) ? w : (T)0;
-}
-
-// ---------------------------------------------------------------------------------------------
-// Fused collide + boundary hook + stream of one level sub-step.
-// ---------------------------------------------------------------------------------------------
-template <typename T, typename S>
-struct StepArgs {
-    const int *ids;
-    int n;
-    const S *A;
-    S *B;
-    long long ncm;
-    const int *nbr_slot;   // per block, Q_max neighbour IDs in 3x3(x3) slot order
-    const int *part;       // block collides and streams (not solid-with-children)
-    const int *simple;     // block and its neighbourhood: all participate, no solid cells
-    const int *cells_mask;
-    const int *onb;
-    T omeg, omegp, U;
-    int mrt;      // collision operator: 0 BGK, 1 MRT
-    T ck[27];     // MRT: rate_k / D_k per moment row (0 for conserved rows)
-    int bc_preset;
-    int *exc_idx;
-    T *exc_val;
-    int *exc_count;
-    long long exc_cap;
-    // Finest-level pairs (3D): vmode 1 -- the exception list (exc_*) is the extra list that the
-    // next sub-step applies as it loads, and each block with an entry gets PEND_FLAG in flags;
-    // vmode 2 -- apply that list (va_*) to the loaded values of flagged blocks; 0 -- neither.
-    int vmode;
-    int *flags;
-    const int *va_idx;
-    const T *va_val;
-    const int *va_count;
-    // The extra list linked per block: x_head[block] is the last node 2k + s of the block's chain
-    // (entry k, s = 0 through its initiator cell, 1 through its partner cell), -1 when empty;
-    // x_next[node] the node before it.  Built in vmode 1, walked and emptied in vmode 2.
-    int *x_head;
-    int *x_next;
-};
-
-// Block flag bit: the block has entries in the finest level's extra exception list (bits 0-1 of
-// the same word hold the simple / interior kind).
-constexpr int PEND_FLAG = 4;
-
-// Appends a guard exception (target cell, partner cell, direction, partner's stored value) to the
-// launch's list; in vmode 1 also flags the two blocks for the next sub-step.
-template <typename T, typename S>
-__device__ __forceinline__ void record_exception(const StepArgs<T, S> &a, long long tgt, long long cell, int q, T fv)
-{
-    int k = atomicAdd(&a.exc_count[0], 1);
-    if (k < a.exc_cap) {
-        a.exc_idx[3 * (long long)k + 0] = (int)tgt;  // cell indices < 2^31
-        a.exc_idx[3 * (long long)k + 1] = (int)cell;
-        a.exc_idx[3 * (long long)k + 2] = q;
-        a.exc_val[k] = fv;
-    } else {
-        a.exc_count[1] = 1;
-    }
-    if (a.vmode == 1) {
-        const int bt = (int)(tgt >> 6), bc = (int)(cell >> 6);
-        atomicOr(&a.flags[bt], PEND_FLAG);
-        atomicOr(&a.flags[bc], PEND_FLAG);
-        if (k < a.exc_cap) {
-            a.x_next[2 * k] = atomicExch(&a.x_head[bt], 2 * k);
-            if (bc != bt) a.x_next[2 * k + 1] = atomicExch(&a.x_head[bc], 2 * k + 1);
-        }
-    }
-}
-
-// Workgroup -> position in the level's block list.  Workgroups are dealt round-robin to the
-// eight XCDs (each with its own L2); giving every XCD one contiguous range of the sorted ID list
-// keeps a block and most of its neighbours -- whose pushes share cache lines -- on one L2.
-__device__ __forceinline__ int xcd_local_wg(int nwg_padded)
-{
-    const int per = nwg_padded / 8;
-    return (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-}
-
-// The same for the first nwg_padded (a multiple of 8) workgroups of a larger grid.
-__device__ __forceinline__ int xcd_local_wg(int wg, int nwg_padded)
-{
-    const int per = nwg_padded / 8;
-    return (wg % 8) * per + wg / 8;
-}
-
-// Post-collision values f*_p of one cell.  BGK: Cu_Collide (solver_lbm_kernels.cu:275-282).  MRT:
-// f* = f - M^T (ck .* (M (f - feq))), the transforms summed in ascending row / column order with
-// zero entries and conserved rows left out (ck_k = rate_k / D_k).  Cells that do not collide
-// (solid cells, blocks that are solid with children) keep their values: the swap semantics of the
-// reference amount to f*_q = f_pb(q) for them.
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void collide_cell(const StepArgs<T, S> &a, const T *f, T *fs, T rho, T u, T v, T w,
-                                             bool inert)
-{
-    using VS = VelSet<Q>;
-    if (inert) {
-#pragma unroll
-        for (int p = 0; p < Q; p++) fs[p] = f[VS::pb(p)];
-        return;
-    }
-    const T udotu = u * u + v * v + w * w;
-    if (!a.mrt) {
-        // BGK in fused multiply-adds, in the same order as the CPU restatement:
-        //   b_p = (4.5 c.u) c.u + (1 - 1.5 u.u),  feq_p / (w_p rho) = 3 c.u + b_p,
-        //   f*_p = (w_p rho omega) (feq_p / (w_p rho)) + (1 - omega) f_p.
-        // A pair (p, pb(p)) shares |c.u|, b and the weight: c_pb.u = -(c_p.u) bit for bit (sums of
-        // negated terms), so the pb direction takes -3 c.u.
-        const T c1 = (T)(1.0) - (T)(1.5) * udotu;
-        const T ro = rho * a.omeg;
-        fs[0] = fmadd((T)VS::w(0) * ro, c1, f[0] * a.omegp);
-#pragma unroll
-        for (int p = 1; p < Q; p++) {
-            if (!VS::half(p)) continue;
-            const int q = VS::pb(p);
-            const T cu = cdot<T, Q>(p, u, v, w);
-            const T b = fmadd((T)(4.5) * cu, cu, c1);
-            const T wro = (T)VS::w(p) * ro;
-            fs[p] = fmadd(wro, fmadd((T)(3.0), cu, b), f[p] * a.omegp);
-            fs[q] = fmadd(wro, fmadd((T)(-3.0), cu, b), f[q] * a.omegp);
-        }
-        return;
-    }
-    using MB = Mrt<Q>;
-    // Full unrolling keeps d, r and the rates in registers (otherwise the FP64 D3Q27 variant indexes
-    // them dynamically from scratch memory).
-    T d[Q];
-#pragma clang loop unroll(full)
-    for (int p = 0; p < Q; p++) {
-        T cdotu = cdot<T, Q>(p, u, v, w);
-        d[p] = f[p] - (T)VS::w(p) * rho * ((T)(1.0) + (T)(3.0) * cdotu + (T)(4.5) * cdotu * cdotu - (T)(1.5) * udotu);
-    }
-    T r[Q];
-#pragma clang loop unroll(full)
-    for (int k = 0; k < Q; k++) {
-        r[k] = (T)0;
-        if (MB::rate(k) == 0) continue;
-        T acc = (T)0;
-        bool first = true;
-#pragma clang loop unroll(full)
-        for (int p = 0; p < Q; p++) {
-            if (MB::m(k, p) == 0) continue;
-            const T term = (T)MB::m(k, p) * d[p];
-            acc = first ? term : acc + term;
-            first = false;
-        }
-        r[k] = acc * a.ck[k];
-    }
-#pragma clang loop unroll(full)
-    for (int p = 0; p < Q; p++) {
-        T acc = (T)0;
-        bool first = true;
-#pragma clang loop unroll(full)
-        for (int k = 0; k < Q; k++) {
-            if (MB::rate(k) == 0 || MB::m(k, p) == 0) continue;
-            const T term = (T)MB::m(k, p) * r[k];
-            acc = first ? term : acc + term;
-            first = false;
-        }
-        fs[p] = f[p] - acc;
-    }
-}
-
-// MRT transform on matrix cores for one 3D block per wavefront (Q = 19, 27; FP32 compute):
-// g = M^T (c . M d) for the non-equilibrium parts d of the 64 cells.  FP32 pools: d and c . M d are
-// split into two bf16 terms each (hi + lo carry 16 significant bits; the products with the integer
-// matrix are exact and the sums FP32), so the result agrees with the vector path to about 2^-17 of
-// d, below the FP32 rounding of the populations themselves.  16-bit pools (F16): one binary16 term
-// of 2^10 d and of 2^10 c . M d each (11 significant bits, the scale keeps small parts out of the
-// subnormal range), products exact and sums FP32, on v_mfma_f32_16x16x32_f16: an error of about
-// 2^-11 of the non-equilibrium part, below the binary16 rounding of the stored deviation f - w,
-// which is larger than that part, and the correction goes back through LDS in binary16.  `lds` is
-// this wavefront's region of 64 rows (36 floats; 80 bytes with 16-bit pools); only the wavefront
-// itself touches it.
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
-
-__constant__ const MfmaTab<19> kMfma19 = make_mfma_tab<19>();
-__constant__ const MfmaTab<27> kMfma27 = make_mfma_tab<27>();
-
-constexpr int MFMA_SPLITS = 2;
-
-// Next bf16 term of `rem` (round to nearest even, the hardware conversion); rem keeps the rest.
-__device__ __forceinline__ __bf16 split_term(float &rem)
-{
-    const __bf16 h = (__bf16)rem;
-    rem -= (float)h;
-    return h;
-}
-
-template <int Q, bool F16>
-__device__ __forceinline__ void mrt_mfma(const float *d, float *g, const float *ckrow, float *lds)
-{
-    using VT = typename std::conditional<F16, f16x8_t, bf16x8_t>::type;
-    constexpr int SPLITS = F16 ? 1 : MFMA_SPLITS;
-    const MfmaTab<Q> &tab = *(Q == 19 ? reinterpret_cast<const MfmaTab<Q> *>(&kMfma19)
-                                      : reinterpret_cast<const MfmaTab<Q> *>(&kMfma27));
-    const int l = threadIdx.x & 63, q = l >> 4, j = l & 15;
-    const u32x4_t *fw = reinterpret_cast<const u32x4_t *>(F16 ? &tab.fw16[l][0][0] : &tab.fw[l][0][0]);
-    const u32x4_t *bk = reinterpret_cast<const u32x4_t *>(F16 ? &tab.bk16[l][0][0] : &tab.bk[l][0][0]);
-    const VT afw0 = __builtin_bit_cast(VT, fw[0]), afw1 = __builtin_bit_cast(VT, fw[1]);
-    const VT abk0 = __builtin_bit_cast(VT, bk[0]), abk1 = __builtin_bit_cast(VT, bk[1]);
-    VT *ldsv = reinterpret_cast<VT *>(lds);  // rows of 5 vectors (80 bytes)
-    auto mfma = [](const VT &a, const VT &b, const f32x4_t &c) {
-        if constexpr (F16)
-            return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-        else
-            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-    };
-    auto term = [](float &rem) {
-        if constexpr (F16) {
-            return (_Float16)rem;
-        } else {
-            return split_term(rem);
-        }
-    };
-
-    // Forward: one pass per term of d through a 64-row transpose region.
-    f32x4_t C0[4], C1[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) C0[t] = C1[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float rem[32];
-#pragma unroll
-    for (int k = 0; k < 32; k++) rem[k] = k < Q ? d[k] : 0.f;
-#pragma unroll
-    for (int sp = 0; sp < SPLITS; sp++) {
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            VT v;
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = term(rem[8 * c + e]);
-            ldsv[5 * l + c] = v;
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const VT b = ldsv[5 * (16 * t + j) + q];
-            C0[t] = mfma(afw0, b, C0[t]);
-            C1[t] = mfma(afw1, b, C1[t]);
-        }
-        wave_lds_sync();
-    }
-    // Relaxation factors rate / D of the rows this lane holds (rows 4q + r and 16 + 4q + r, zero
-    // beyond the velocity set), picked from the level's row table by the lane's quarter q.
-    float ck0[4], ck1[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        float a0[4], a1[4];
-#pragma unroll
-        for (int qq = 0; qq < 4; qq++) {
-            a0[qq] = 4 * qq + r < Q ? ckrow[4 * qq + r] : 0.f;
-            a1[qq] = 16 + 4 * qq + r < Q ? ckrow[16 + 4 * qq + r] : 0.f;
-        }
-        ck0[r] = q == 0 ? a0[0] : (q == 1 ? a0[1] : (q == 2 ? a0[2] : a0[3]));
-        ck1[r] = q == 0 ? a1[0] : (q == 1 ? a1[1] : (q == 2 ? a1[2] : a1[3]));
-    }
-    // Back: B operand straight from the forward results of the same lane.
-    f32x4_t G0[4], G1[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        G0[t] = G1[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        float v[8];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            v[r] = C0[t][r] * ck0[r];
-            v[4 + r] = C1[t][r] * ck1[r];
-        }
-#pragma unroll
-        for (int sp = 0; sp < SPLITS; sp++) {
-            VT b;
-#pragma unroll
-            for (int e = 0; e < 8; e++) b[e] = term(v[e]);
-            G0[t] = mfma(abk0, b, G0[t]);
-            G1[t] = mfma(abk1, b, G1[t]);
-        }
-    }
-    if constexpr (F16) {
-        // Transpose back in binary16 (the scaled correction, 11 significant bits, far below the
-        // storage step of the deviation it corrects): rows of 40 halves (80 bytes) per cell.
-        typedef __attribute__((ext_vector_type(4))) _Float16 f16x4_t;
-        _Float16 *ldsh = reinterpret_cast<_Float16 *>(lds);
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            f16x4_t a, b;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                a[r] = (_Float16)G0[t][r];
-                b[r] = (_Float16)G1[t][r];
-            }
-            *reinterpret_cast<f16x4_t *>(ldsh + 40 * (16 * t + j) + 4 * q) = a;
-            *reinterpret_cast<f16x4_t *>(ldsh + 40 * (16 * t + j) + 16 + 4 * q) = b;
-        }
-        wave_lds_sync();
-        const f16x8_t *row = reinterpret_cast<const f16x8_t *>(ldsh + 40 * l);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const f16x8_t h = row[c];
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                if (8 * c + e < Q) g[8 * c + e] = (float)h[e];
-        }
-        wave_lds_sync();
-    } else {
-        // Transpose back: G row p of cell 16t + j -> LDS row of that cell (36 floats), then own row.
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            *reinterpret_cast<f32x4_t *>(lds + 36 * (16 * t + j) + 4 * q) = G0[t];
-            *reinterpret_cast<f32x4_t *>(lds + 36 * (16 * t + j) + 16 + 4 * q) = G1[t];
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int p = 0; p < Q; p++) g[p] = lds[36 * l + p];
-        wave_lds_sync();
-    }
-}
-
-// Population load of the fused step.  FP32/FP64 rows are read with non-temporal loads: they are
-// used once, and keeping them out of L2 leaves it to the pushes, whose partial cache lines from
-// neighbouring blocks merge there (measured: the FP32 fused step runs ~20% faster).  16-bit rows
-// measured slightly slower that way and use ordinary loads.
-template <typename S>
-__device__ __forceinline__ S load_pop(const S *p)
-{
-    if constexpr (sizeof(S) >= 4)
-        return __builtin_nontemporal_load(p);
-    else
-        return *p;
-}
-
-template <typename S>
-__device__ __forceinline__ S load_pop(const __attribute__((address_space(1))) S *p)
-{
-    if constexpr (sizeof(S) >= 4)
-        return __builtin_nontemporal_load(p);
-    else if constexpr (std::is_same<S, bf16s>::value)
-        return bf16s{*reinterpret_cast<const __attribute__((address_space(1))) uint16_t *>(p)};
-    else
-        return *p;
-}
-
-// A global-memory pointer that is the same on every lane, forced into scalar registers: a lane's
-// element of it is then a scalar base plus a 32-bit offset, with no 64-bit vector address
-// arithmetic per access.
-template <typename S>
-__device__ __forceinline__ const __attribute__((address_space(1))) S *scalar_row(const S *p)
-{
-    const unsigned long long v = reinterpret_cast<unsigned long long>(p);
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-    return (const __attribute__((address_space(1))) S *)(((unsigned long long)hi << 32) | lo);
-}
-
-// Store of the fused step into a row (the same pointer on every lane) at element idx.  A 16-bit
-// row holds fewer than 2^32 bytes (the pool has fewer than 2^31 cells, checked at creation), so the
-// address is a scalar base plus a 32-bit byte offset, with no 64-bit vector address arithmetic per
-// store; wider rows keep 64-bit addresses.
-template <typename S>
-__device__ __forceinline__ void store_pop(S *row, unsigned idx, S v)
-{
-    if constexpr (sizeof(S) == 2) {
-        const unsigned long long r = reinterpret_cast<unsigned long long>(row);
-        const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)r), hi = __builtin_amdgcn_readfirstlane((unsigned)(r >> 32));
-        auto *base = (__attribute__((address_space(1))) char *)(((unsigned long long)hi << 32) | lo);
-        *(__attribute__((address_space(1))) uint16_t *)(base + idx * 2u) = __builtin_bit_cast(uint16_t, v);
-    } else {
-        row[idx] = v;
-    }
-}
-
-// Store of a 16-bit value at a byte offset within a row (the same pointer on every lane).
-template <typename S>
-__device__ __forceinline__ void store_pop_bytes(S *row, unsigned byte_off, S v)
-{
-    static_assert(sizeof(S) == 2, "16-bit rows only");
-    const unsigned long long r = reinterpret_cast<unsigned long long>(row);
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)r), hi = __builtin_amdgcn_readfirstlane((unsigned)(r >> 32));
-    auto *base = (__attribute__((address_space(1))) char *)(((unsigned long long)hi << 32) | lo);
-    *(__attribute__((address_space(1))) uint16_t *)(base + byte_off) = __builtin_bit_cast(uint16_t, v);
-}
-
-// One link of the fused step for the cell `cell`, direction q >= 1, whose neighbour block in that
-// direction is nbk (target cell tgt): boundary hook, swap guard, and the single store of f*_q
-// either into the neighbour (the link streams) or into the cell's own opposite slot (bounce-back).
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void push_link(const StepArgs<T, S> &a, int q, T fq, int nbk, long long tgt, long long cell,
-                                          bool inert, bool simple, bool onb, T u, T v, T w)
-{
-    using VS = VelSet<Q>;
-    using ST = Store<T, S>;
-    // Domain-face hook on links that leave the domain (Cu_ImposeBC, onb blocks, non-solid cells).
-    if (onb && nbk < 0 && nbk != N_SKIPID)
-        fq = bc_hook<T>(a.bc_preset, a.U, nbk, fq, u, v, w, (T)VS::w(q), (T)VS::cx(q), (T)VS::cy(q), (T)VS::cz(q));
-    // In a 16-bit pool the guard below sees the stored value.
-    fq = quant<T, S>(fq, (T)VS::w(q));
-    bool push;
-    bool exc = false;
-    if (VS::half(q)) {
-        // Initiator of the link x -> x + c_q.
-        push = !inert && nbk >= 0;
-        if (!simple && push) {
-            const bool p_inert = !a.part[nbk] || a.cells_mask[tgt] == CELL_SOLID;
-            if (p_inert) push = ST::dec(a.A[(long long)q * a.ncm + tgt], (T)VS::w(q)) > (T)0;
-        }
-    } else {
-        // Partner of the link initiated by the cell x + c_q in direction pb(q).
-        push = nbk >= 0;
-        if (!simple && push) push = a.part[nbk] && a.cells_mask[tgt] != CELL_SOLID;
-        if (push && !(fq > (T)0)) {
-            push = false;
-            exc = !inert;  // a colliding partner cannot tell the initiator in time
-        }
-    }
-    if (exc) {
-        record_exception(a, tgt, cell, q, fq);
-        return;
-    }
-    const long long at = push ? (long long)q * a.ncm + tgt : (long long)VS::pb(q) * a.ncm + cell;
-    a.B[at] = ST::enc(fq, (T)VS::w(q));
-}
-
-// Stream of an interior block (block flag simple == 2): every neighbour slot of the velocity set
-// exists, and the block and its neighbours participate with no solid cell.  No link then leaves
-// the domain or the level, no guard read is needed, half-set links always push, and the partner
-// side pushes unless its stored value fails the guard (then the link goes to the exception list,
-// as in push_link).  The target block comes from the wave's neighbour table (lane s holds slot s)
-// through ds_bpermute; the target cell from a carry-free add of the link to the lane's (I,J,K)
-// 2-bit fields.  Same stores, same values as push_link on these blocks, with about a fifth of its
-// vector instructions.
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void push_interior(const StepArgs<T, S> &a, const T *fs, int my_nb, int t, unsigned cell)
-{
-    using VS = VelSet<Q>;
-    using ST = Store<T, S>;
-    const int I = t & 3, J = (t >> 2) & 3, K = t >> 4;
-    // ds_bpermute byte steps to the neighbour slot along each axis, nonzero on the block's faces.
-    const int xp = I == 3 ? 4 : 0, xm = I == 0 ? -4 : 0;
-    const int yp = J == 3 ? 12 : 0, ym = J == 0 ? -12 : 0;
-    const int zp = K == 3 ? 36 : 0, zm = K == 0 ? -36 : 0;
-    // 16-bit rows: the target as a byte offset within the row (block << 7 | cell << 1), the same
-    // field-wise sum on fields shifted up by one bit, so the store needs no further shift.
-    constexpr int SH = sizeof(S) == 2 ? 1 : 0;
-    const unsigned tl = ((unsigned)t & 0x15u) << SH, th = ((unsigned)t & 0x2Au) << SH;
-    const int nb_src = (int)((unsigned)my_nb << (6 + SH));
-#pragma unroll
-    for (int q = 1; q < Q; q++) {
-        const int cx = VS::cx(q), cy = VS::cy(q), cz = VS::cz(q);
-        int sa = 13 * 4;
-        if (cx > 0) sa += xp;
-        if (cx < 0) sa += xm;
-        if (cy > 0) sa += yp;
-        if (cy < 0) sa += ym;
-        if (cz > 0) sa += zp;
-        if (cz < 0) sa += zm;
-        const unsigned nbk = (unsigned)__builtin_amdgcn_ds_bpermute(sa, nb_src);
-        // ((I+cx)&3) + 4((J+cy)&3) + 16((K+cz)&3): field-wise sum without carries between fields.
-        const unsigned d = (unsigned)((cx & 3) | ((cy & 3) << 2) | ((cz & 3) << 4));
-        const unsigned tgt_s = nbk + ((tl + ((d & 0x15u) << SH)) ^ th ^ ((d & 0x2Au) << SH));
-        const S e = ST::enc(fs[q], (T)VS::w(q));
-        bool push = true;
-        if (!VS::half(q)) {
-            // Partner of the link initiated by the cell x + c_q: the guard on the stored value.
-            if (!ST::positive(e, (T)VS::w(q))) {
-                push = false;
-                record_exception(a, (long long)(tgt_s >> SH), (long long)cell, q, ST::dec(e, (T)VS::w(q)));
-            }
-        }
-        if (push) {
-            if constexpr (SH == 1)
-                store_pop_bytes(a.B + (long long)q * a.ncm, tgt_s, e);
-            else
-                store_pop(a.B + (long long)q * a.ncm, tgt_s, e);
-        }
-    }
-}
-
-// Stream of a simple block that is not interior (block flag simple == 1): the block and its
-// existing neighbours participate with no solid cell, but some neighbour slots are missing (a
-// domain face, or a coarser region).  Same lookup and target arithmetic as push_interior; a link
-// whose neighbour slot is missing bounces back into the cell's own opposite slot, after the face
-// hook when the block lies on the domain boundary (onb) and the slot is a face -- push_link's
-// rules for non-inert cells of simple blocks.
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void push_simple(const StepArgs<T, S> &a, const T *fs, int my_nb, int t, unsigned cell,
-                                            bool onb, T u, T v, T w)
-{
-    using VS = VelSet<Q>;
-    using ST = Store<T, S>;
-    const int I = t & 3, J = (t >> 2) & 3, K = t >> 4;
-    const int xp = I == 3 ? 4 : 0, xm = I == 0 ? -4 : 0;
-    const int yp = J == 3 ? 12 : 0, ym = J == 0 ? -12 : 0;
-    const int zp = K == 3 ? 36 : 0, zm = K == 0 ? -36 : 0;
-    const unsigned tl = (unsigned)t & 0x15u, th = (unsigned)t & 0x2Au;
-#pragma unroll
-    for (int q = 1; q < Q; q++) {
-        const int cx = VS::cx(q), cy = VS::cy(q), cz = VS::cz(q);
-        int sa = 13 * 4;
-        if (cx > 0) sa += xp;
-        if (cx < 0) sa += xm;
-        if (cy > 0) sa += yp;
-        if (cy < 0) sa += ym;
-        if (cz > 0) sa += zp;
-        if (cz < 0) sa += zm;
-        const int nbk = __builtin_amdgcn_ds_bpermute(sa, my_nb);
-        const unsigned d = (unsigned)((cx & 3) | ((cy & 3) << 2) | ((cz & 3) << 4));
-        const unsigned tgt = ((unsigned)nbk << 6) + ((tl + (d & 0x15u)) ^ th ^ (d & 0x2Au));
-        T fq = fs[q];
-        if (onb && nbk < 0 && nbk != N_SKIPID)
-            fq = bc_hook<T>(a.bc_preset, a.U, nbk, fq, u, v, w, (T)VS::w(q), (T)VS::cx(q), (T)VS::cy(q), (T)VS::cz(q));
-        const S e = ST::enc(fq, (T)VS::w(q));
-        bool push = nbk >= 0;
-        if (!VS::half(q) && push) {
-            // Partner of the link initiated by the cell x + c_q: the guard on the stored value.
-            if (!ST::positive(e, (T)VS::w(q))) {
-                record_exception(a, (long long)tgt, (long long)cell, q, ST::dec(e, (T)VS::w(q)));
-                continue;  // no store: the fixup places both values
-            }
-        }
-        if (push)
-            store_pop(a.B + (long long)q * a.ncm, tgt, e);
-        else
-            store_pop(a.B + (long long)VS::pb(q) * a.ncm, cell, e);
-    }
-}
-
-// The extra exception list of the previous finest sub-step, applied to this block's loaded values:
-// for an entry (initiator cell i, partner cell c, direction q) the fixup would move the value at
-// (pb(q), c) -- the initiator's push -- to (q, i) and store the partner's value at (pb(q), c).
-// The previous sub-step's output is this sub-step's input, read by no one else in between, so
-// the same values are taken here as the loads' results instead.  No two entries share a slot (an
-// entry's q is the partner's, non-initiating direction and pb(q) an initiating one), so the order
-// of application is free.  The wavefront walks its block's chain (the entries with i or c in the
-// block, linked when they were recorded), so the work per block is its own entries however long
-// the list is; the chain is emptied for the next pair.
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void apply_pending(const StepArgs<T, S> &a, T *f, int b, int t)
-{
-    using VS = VelSet<Q>;
-    using ST = Store<T, S>;
-    const unsigned my = ((unsigned)b << 6) | (unsigned)t;
-    int e = __builtin_amdgcn_readfirstlane(a.x_head[b]);
-    while (e >= 0) {
-        const int k = e >> 1;
-        const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane(a.va_idx[3 * (long long)k + 0]);
-        const unsigned hc = (unsigned)__builtin_amdgcn_readfirstlane(a.va_idx[3 * (long long)k + 1]);
-        const int hq = __builtin_amdgcn_readfirstlane(a.va_idx[3 * (long long)k + 2]);
-        int qb = 0;
-        T wq = 0;
-#pragma unroll
-        for (int p = 0; p < Q; p++)
-            if (p == hq) {
-                qb = VS::pb(p);
-                wq = (T)VS::w(p);
-            }
-        // Through storage, as the fixup's store and this sub-step's load would take them.
-        const T vi = ST::dec(a.A[(long long)qb * a.ncm + hc], wq);
-        const T vc = ST::dec(ST::enc(a.va_val[k], wq), wq);
-        const bool at_i = hi == my, at_c = hc == my;
-#pragma unroll
-        for (int p = 1; p < Q; p++) {
-            if (at_i && p == hq) f[p] = vi;
-            if (at_c && p == qb) f[p] = vc;
-        }
-        e = __builtin_amdgcn_readfirstlane(a.x_next[e]);
-    }
-    if (t == 0) a.x_head[b] = -1;
-}
-
-// 3D: one wavefront per block, so the block, its flags and its 27 neighbour IDs are wave-uniform
-// (scalar registers); each lane picks its link's neighbour among at most eight of them with
-// selects on its own cell position -- no LDS traffic and no per-direction waits.  Interior blocks
-// take push_interior instead.
-template <typename T, typename S, int Q, bool MF>
-__device__ __forceinline__ void collide_stream_3d(const StepArgs<T, S> &a, int wave, float *lds)
-{
-    using VS = VelSet<Q>;
-    using ST = Store<T, S>;
-    const int t = threadIdx.x & 63;
-    const int bi = wave;  // one block per wavefront
-    if (bi >= a.n) return;  // whole wavefronts only; the kernel has no barrier
-    const int b = __builtin_amdgcn_readfirstlane(a.ids[bi]);
-    // Cell index within a population row (the pool holds fewer than 2^32 cells, checked at
-    // creation), so rows are addressed as a row base plus a 32-bit index.
-    const unsigned cell = (unsigned)b * 64u + (unsigned)t;
-    // Lane s < 27 holds neighbour slot s (lanes above repeat slot 26): a load on every lane keeps
-    // the block index out of divergent control flow, so it stays a scalar.
-    const int my_nb = a.nbr_slot[(long long)b * 27 + (t < 27 ? t : 26)];
-    const int flags_u = __builtin_amdgcn_readfirstlane(a.simple[b]);
-    if (flags_u & LINK_FLAG) return;  // a linked block: its sub-step is k_link_step's
-    const int simple_u = flags_u & 3;
-    const int part_u = __builtin_amdgcn_readfirstlane(a.part[b]);
-    const int onb_u = __builtin_amdgcn_readfirstlane(a.onb[b]);
-    T f[Q];
-#pragma unroll
-    for (int q = 0; q < Q; q++)  // row q of block b: a scalar base, lane t at offset t
-        f[q] = ST::dec(load_pop(scalar_row(a.A + (long long)q * a.ncm + (long long)b * 64) + t), (T)VS::w(q));
-    if (a.vmode == 2 && (flags_u & PEND_FLAG)) {
-        apply_pending<T, S, Q>(a, f, b, t);
-        if (t == 0) a.flags[b] = simple_u;  // this sub-step sets no flags: no other writer
-    }
-    const bool simple = simple_u != 0;
-    int mask = CELL_INTERIOR;
-    if (!simple) mask = a.cells_mask[cell];
-    const bool inert = part_u == 0 || mask == CELL_SOLID;
-    const bool onb = onb_u == 1 && mask != CELL_SOLID;
-
-    T fs[Q];
-    T rho, u, v, w;
-    moments<T, Q>(f, rho, u, v, w);
-    if constexpr (MF) {
-        // MRT with the moment transform on matrix cores (whole wavefront, inert lanes carry zeros).
-        // The non-equilibrium parts go in scaled by SC (16-bit pools: 2^10, see mrt_mfma) and the
-        // correction comes back scaled by SC; the equilibrium in pairs (p, pb(p)) with fused
-        // multiply-adds, SC folded into the density.
-        constexpr float SC = ST::quantized ? 1024.0f : 1.0f;
-        const T c1 = (T)(1.0) - (T)(1.5) * (u * u + v * v + w * w);
-        const T rs = rho * (T)SC;
-        float d[Q], g[Q];
-        d[0] = inert ? 0.f : fmadd(f[0], (T)SC, -((T)VS::w(0) * rs * c1));
-#pragma unroll
-        for (int p = 1; p < Q; p++) {
-            if (!VS::half(p)) continue;
-            const int q = VS::pb(p);
-            const T cu = cdot<T, Q>(p, u, v, w);
-            const T b = fmadd((T)(4.5) * cu, cu, c1);
-            const T wr = (T)VS::w(p) * rs;
-            d[p] = inert ? 0.f : fmadd(f[p], (T)SC, -(wr * fmadd((T)(3.0), cu, b)));
-            d[q] = inert ? 0.f : fmadd(f[q], (T)SC, -(wr * fmadd((T)(-3.0), cu, b)));
-        }
-        mrt_mfma<Q, ST::quantized>(d, g, a.ck, lds);
-#pragma unroll
-        for (int p = 0; p < Q; p++) fs[p] = inert ? f[VS::pb(p)] : fmadd((T)g[p], (T)(-1.0f / SC), f[p]);
-    } else {
-        collide_cell<T, S, Q>(a, f, fs, rho, u, v, w, inert);
-    }
-
-    store_pop(a.B, cell, ST::enc(fs[0], (T)VS::w(0)));
-    if (simple_u == 2) {
-        push_interior<T, S, Q>(a, fs, my_nb, t, cell);
-        return;
-    }
-    if (simple_u == 1) {
-        push_simple<T, S, Q>(a, fs, my_nb, t, cell, onb_u == 1, u, v, w);
-        return;
-    }
-    int nbs[27];
-#pragma unroll
-    for (int s = 0; s < 27; s++) nbs[s] = __builtin_amdgcn_readlane(my_nb, s);
-    const int I = t & 3, J = (t >> 2) & 3, K = t >> 4;
-#pragma unroll
-    for (int q = 1; q < Q; q++) {
-        const int cx = VS::cx(q), cy = VS::cy(q), cz = VS::cz(q);
-        // Does the link leave the block along x / y / z?
-        const bool ex = cx > 0 ? I == 3 : (cx < 0 ? I == 0 : false);
-        const bool ey = cy > 0 ? J == 3 : (cy < 0 ? J == 0 : false);
-        const bool ez = cz > 0 ? K == 3 : (cz < 0 ? K == 0 : false);
-        // Slot (dx+1) + 3(dy+1) + 9(dz+1) of the neighbour block; 13 is the block itself.
-        const int sxyz = nbs[13 + cx + 3 * cy + 9 * cz], sxy = nbs[13 + cx + 3 * cy], sxz = nbs[13 + cx + 9 * cz],
-                  syz = nbs[13 + 3 * cy + 9 * cz], sx = nbs[13 + cx], sy = nbs[13 + 3 * cy], sz = nbs[13 + 9 * cz];
-        const int nbk = ex ? (ey ? (ez ? sxyz : sxy) : (ez ? sxz : sx)) : (ey ? (ez ? syz : sy) : (ez ? sz : b));
-        const long long tgt = (long long)nbk * 64 + (((I + cx) & 3) + 4 * ((J + cy) & 3) + 16 * ((K + cz) & 3));
-        push_link<T, S, Q>(a, q, fs[q], nbk, tgt, (long long)cell, inert, simple, onb, u, v, w);
-    }
-}
-
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void collide_stream_2d(const StepArgs<T, S> &a, int wave);
-
-// One launch of the fused step over the blocks of up to MAXLV levels: the levels' wavefront slots
-// are consecutive ranges [start[k], start[k+1]) of the launch (one 3D block or four 2D blocks per
-// slot), dealt to the XCDs in contiguous ranges.  Levels of one launch touch disjoint cells and
-// their own exception lists, so one launch does what separate launches of each level would.
-constexpr int MAXLV = 4;
-
-template <typename T, typename S>
-struct MultiStep {
-    int nlv;
-    int start[MAXLV + 1];
-    StepArgs<T, S> lv[MAXLV];
-};
-
-// 2D: four 4x4 blocks per wavefront; neighbour IDs are distributed with ds_bpermute.
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void collide_stream_2d(const StepArgs<T, S> &a, int wave)
-{
-    using VS = VelSet<Q>;
-    using ST = Store<T, S>;
-    constexpr int CELLS = VS::CELLS, DIM = VS::DIM, QMAX = VS::QMAX;
-    const int t = threadIdx.x % CELLS;
-    const int lane = threadIdx.x % 64;
-    const int gbase = lane - t;  // lane of cell 0 of this block within the wavefront
-    const int bi = wave * (64 / CELLS) + lane / CELLS;
-    const bool active = bi < a.n;
-    const int b = active ? a.ids[bi] : 0;
-    // Lane-parallel load of the block's neighbour table; distributed with ds_bpermute (every
-    // __shfl below sits outside divergent control flow).
-    const int my_nb = (active && t < QMAX) ? a.nbr_slot[(long long)b * QMAX + t] : N_SKIPID;
-    const int I = t % 4, J = (t / 4) % 4, K = (DIM == 3) ? t / 16 : 0;
-    const long long cell = (long long)b * CELLS + t;
-
-    bool simple = true, inert = false, onb = false;
-    int mask = CELL_INTERIOR;
-    T f[Q];
-    if (active) {
-        simple = (a.simple[b] & 3) != 0;
-        const bool part = a.part[b] != 0;
-        if (!simple) mask = a.cells_mask[cell];
-        inert = !part || mask == CELL_SOLID;
-        onb = a.onb[b] == 1 && mask != CELL_SOLID;
-#pragma unroll
-        for (int q = 0; q < Q; q++) f[q] = ST::dec(load_pop(&a.A[(long long)q * a.ncm + cell]), (T)VS::w(q));
-    } else {
-#pragma unroll
-        for (int q = 0; q < Q; q++) f[q] = (T)1;
-    }
-
-    T fs[Q];
-    T rho, u, v, w;
-    moments<T, Q>(f, rho, u, v, w);
-    collide_cell<T, S, Q>(a, f, fs, rho, u, v, w, inert);
-
-    if (active) a.B[cell] = ST::enc(fs[0], (T)VS::w(0));
-#pragma unroll
-    for (int q = 1; q < Q; q++) {
-        const int Ip = I + VS::cx(q), Jp = J + VS::cy(q), Kp = K + VS::cz(q);
-        const int slot = (Ip < 0 ? 0 : (Ip >= 4 ? 2 : 1)) + 3 * (Jp < 0 ? 0 : (Jp >= 4 ? 2 : 1)) +
-                         (DIM == 3 ? 9 * (Kp < 0 ? 0 : (Kp >= 4 ? 2 : 1)) : 0);
-        const int nbk = __shfl(my_nb, gbase + slot, 64);
-        if (!active) continue;
-        const long long tgt = (long long)nbk * CELLS + ((Ip & 3) + 4 * (Jp & 3) + (DIM == 3 ? 16 * (Kp & 3) : 0));
-        push_link<T, S, Q>(a, q, fs[q], nbk, tgt, cell, inert, simple, onb, u, v, w);
-    }
-}
-
-// Resolves guard exceptions: the initiator's pushed value returns to it (bounce-back) and the
-// partner keeps its own post-collision value.  One workgroup per level of the fused launch, each on
-// its level's list; it clears the list's counter when done.
-template <typename T, typename S>
-struct FixupArgs {
-    long long ncm, exc_cap;
-    S *B[MAXLV];
-    const int *exc_idx[MAXLV];
-    const T *exc_val[MAXLV];
-    int *exc_count[MAXLV];
-    int *va_count[MAXLV];  // the finest level: its extra list's counter, cleared here, else null
-};
-
-template <typename T, typename S, int Q>
-__device__ __forceinline__ void fixup_level(const FixupArgs<T, S> &fa, int lv)
-{
-    using VS = VelSet<Q>;
-    S *__restrict__ B = fa.B[lv];
-    const int *__restrict__ exc_idx = fa.exc_idx[lv];
-    const T *__restrict__ exc_val = fa.exc_val[lv];
-    int *exc_count = fa.exc_count[lv];
-    const long long ncm = fa.ncm;
-    // The extra list was applied by the sub-step that this list comes from; it starts empty for the
-    // next pair.
-    if (fa.va_count[lv] && threadIdx.x == 0 && fa.va_count[lv][0] != 0) fa.va_count[lv][0] = 0;
-    const int cnt = exc_count[0];
-    if (cnt == 0) return;  // the usual case: nothing to resolve, nothing to reset (whole workgroup)
-    const long long n = min((long long)cnt, fa.exc_cap);
-    for (long long k = threadIdx.x; k < n; k += WG) {
-        const long long i = (unsigned)exc_idx[3 * k + 0], c = (unsigned)exc_idx[3 * k + 1];
-        const int q = exc_idx[3 * k + 2];
-        int qb = 0;
-        T wq = 0;
-#pragma unroll
-        for (int p = 0; p < Q; p++)
-            if (p == q) {
-                qb = VS::pb(p);
-                wq = (T)VS::w(p);
-            }
-        // Rows q and pb(q) share one weight: a stored value moves between them unchanged.
-        B[(long long)q * ncm + i] = B[(long long)qb * ncm + c];
-        B[(long long)qb * ncm + c] = Store<T, S>::enc(exc_val[k], wq);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) exc_count[0] = 0;
-}
-
-template <typename T, typename S, int Q>
-__global__ __launch_bounds__(WG) void k_fixup(FixupArgs<T, S> fa)
-{
-    fixup_level<T, S, Q>(fa, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1111,14 +267,15 @@ __device__ __forceinline__ void group_sums(const T *v, T *acc, T *lds)
 // the averaged values go to the pool and, as the pool will hold them, to LDS, from where the
 // interpolation stage takes them.  Arithmetic and order are those of k_average and k_interp.
 // ---------------------------------------------------------------------------------------------
-template <typename T, typename S, int Q>
-__global__ __launch_bounds__(IWG) void k_avg_interp(const int *__restrict__ ids, int n, S *__restrict__ Fp,
-                                                    S *__restrict__ Fc, long long ncm, const int *__restrict__ nbr_child,
+template <typename T, typename S, int Q, bool FOLD>
+__global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const int *__restrict__ ids, int n, S *Fp, S *Fc,
+                                                    long long ncm, const int *__restrict__ nbr_child,
                                                     const int *__restrict__ blk_mask, const int *__restrict__ cells_mask,
                                                     T ratio_avg, T ratio_int)
 {
     using VS = VelSet<Q>;
     using ST = Store<T, S>;
+    if constexpr (FOLD) resolve_pending<T, S, Q>(fa);
     constexpr int CELLS = VS::CELLS, DIM = VS::DIM, NCH = VS::CHILDREN, HALF = NCH / 2;
     constexpr int GROUP = HALF * CELLS;  // lanes per parent
     constexpr int PPW = IWG / GROUP;     // parents per workgroup
@@ -1451,13 +608,14 @@ __global__ __launch_bounds__(CWG) void k_interp_cubic(InterpArgs<T, S> ia)
 // parent cells (t and t + CELLS/2, both loaded before either is reduced), which halves the
 // wavefronts per parent.  No LDS, no barriers.
 // ---------------------------------------------------------------------------------------------
-template <typename T, typename S, int Q>
-__global__ __launch_bounds__(WG) void k_average(const int *__restrict__ ids, int n, S *__restrict__ Fp,
-                                                const S *__restrict__ Fc, long long ncm, const int *__restrict__ nbr_child,
+template <typename T, typename S, int Q, bool FOLD>
+__global__ __launch_bounds__(WG) void k_average(FixupArgs<T, S> fa, const int *__restrict__ ids, int n, S *Fp,
+                                                const S *Fc, long long ncm, const int *__restrict__ nbr_child,
                                                 const int *__restrict__ blk_mask, const int *__restrict__ cells_mask,
                                                 int ave_type, T tau_ratio)
 {
     using VS = VelSet<Q>;
+    if constexpr (FOLD) resolve_pending<T, S, Q>(fa);
     constexpr int CELLS = VS::CELLS, DIM = VS::DIM;
     constexpr int NG = (DIM == 3) ? 8 : 4;     // child cells per parent cell
     constexpr int PER_BLOCK = CELLS / 2 * NG;   // lanes per parent block: two parent cells per lane group
@@ -1531,30 +689,30 @@ __global__ __launch_bounds__(WG) void k_average(const int *__restrict__ ids, int
 }
 
 // ---------------------------------------------------------------------------------------------
-// The fused step's launch.  The first interp_wgs workgroups interpolate one level's interface
-// parents into their children (k_interp, INTERFACE mode), the next fix_wgs resolve the exception
-// lists of levels that an earlier launch left (k_fixup), and from `lead` on (those two counts
-// rounded up to a multiple of 8, so that the XCD mapping below still deals contiguous ranges)
-// step_wgs workgroups run the fused step of the MultiStep levels.  The few, latency-bound
-// interpolation workgroups go first so that they run beside the fused step instead of after it.
-// The three parts touch disjoint cells: a level's interpolation reads the level's current buffer
-// and writes the finer level's ghost cells, and the launcher hands over only fixups of levels that
-// none of the other parts touches.
+// The fused step's launch.  After the pending exception lists are resolved, the first interp_wgs
+// workgroups interpolate one level's interface parents into their children (k_interp, INTERFACE mode),
+// and from `lead` on (that count rounded up to a multiple of 8, so that the XCD mapping below still
+// deals contiguous ranges) step_wgs workgroups run the fused step of the MultiStep levels.  The few,
+// latency-bound interpolation workgroups go first so that they run beside the fused step instead of
+// after it.  The two parts touch disjoint cells: a level's interpolation reads the level's current
+// buffer and writes the finer level's ghost cells.
 // ---------------------------------------------------------------------------------------------
 template <typename T, typename S>
 struct StepExtras {
-    int step_wgs, interp_wgs, fix_wgs, lead;
+    int step_wgs, interp_wgs, lead;
     InterpArgs<T, S> ia;
     FixupArgs<T, S> fa;
 };
 
 static_assert(IWG == WG, "interpolation and fused-step workgroups share one launch");
 
-template <typename T, typename S, int Q, bool MF>
-__global__ __launch_bounds__(WG) void k_collide_stream(MultiStep<T, S> m, StepExtras<T, S> x)
+// (D3Q27 MRT in FP32 is held to five wavefronts per SIMD: 102 registers without it, four.)
+template <typename T, typename S, int Q, int COLL, bool FOLD>
+__global__ __launch_bounds__(WG, (COLL == COLL_MRT && Q == 27 && sizeof(T) == 4 ? 5 : 1)) void k_collide_stream(MultiStep<T, S> m, StepExtras<T, S> x)
 {
     using VS = VelSet<Q>;
     using IL = InterpLds<T, Q>;
+    constexpr bool MF = COLL == COLL_MFMA;
     // One LDS region shared by the two workgroup kinds of the launch: the interpolation's parent
     // rows and coefficients, or the matrix-core MRT's per-wavefront transpose rows.
     constexpr int ROW = Store<T, S>::quantized ? 20 : 36;
@@ -1562,14 +720,12 @@ __global__ __launch_bounds__(WG) void k_collide_stream(MultiStep<T, S> m, StepEx
     constexpr size_t INTERP_BYTES = sizeof(T) * (ALL16 + IL::COEF);
     constexpr size_t MRT_BYTES = MF ? sizeof(float) * (WG / 64) * 64 * ROW : 0;
     __shared__ __attribute__((aligned(16))) unsigned char s_raw[INTERP_BYTES > MRT_BYTES ? INTERP_BYTES : MRT_BYTES];
+    if constexpr (FOLD) resolve_pending<T, S, Q>(x.fa);
     if ((int)blockIdx.x < x.lead) {
-        const int w2 = blockIdx.x;
-        if (w2 < x.interp_wgs) {
+        if ((int)blockIdx.x < x.interp_wgs) {
             T *s_all = reinterpret_cast<T *>(s_raw);
             T *s_coef = s_all + ALL16;
-            interp_parents<T, S, Q, false>(x.ia, w2, s_all, s_coef);
-        } else if (w2 < x.interp_wgs + x.fix_wgs) {
-            fixup_level<T, S, Q>(x.fa, w2 - x.interp_wgs);
+            interp_parents<T, S, Q, false>(x.ia, blockIdx.x, s_all, s_coef);
         }
         return;
     }
@@ -1583,15 +739,16 @@ __global__ __launch_bounds__(WG) void k_collide_stream(MultiStep<T, S> m, StepEx
     k = __builtin_amdgcn_readfirstlane(k);
     const StepArgs<T, S> &a = m.lv[k];
     const int wave = slot - m.start[k];
-    if constexpr (MF) {
+    if constexpr (VS::DIM == 3) {
         // One transpose region per wavefront for the matrix-core MRT: 64 rows of 36 floats, or of
         // 20 floats (80 bytes: the forward rows, and the back rows in binary16) with 16-bit pools.
-        float *s_mrt = reinterpret_cast<float *>(s_raw);
-        collide_stream_3d<T, S, Q, true>(a, wave, s_mrt + (threadIdx.x >> 6) * 64 * ROW);
-    } else if constexpr (VS::DIM == 3) {
-        collide_stream_3d<T, S, Q, false>(a, wave, nullptr);
+        float *s_mrt = MF ? reinterpret_cast<float *>(s_raw) + (threadIdx.x >> 6) * 64 * ROW : nullptr;
+        if (a.vmode == VMODE_EVEN)
+            even_step_3d<T, S, Q, COLL>(a, wave, s_mrt);
+        else
+            collide_stream_3d<T, S, Q, COLL>(a, wave, s_mrt);
     } else {
-        collide_stream_2d<T, S, Q>(a, wave);
+        collide_stream_2d<T, S, Q, COLL>(a, wave);
     }
 }
 
@@ -1680,7 +837,11 @@ __device__ __forceinline__ void mea_add(T *acc, int order, T f, T fm, float dist
     }
 }
 
-template <typename T, typename S, int Q>
+// FM: the values behind the cells, f*_p(x - c_p), are needed (interpolated bounce-back, or the
+// second-order momentum exchange).  Neighbour blocks are looked up through the wave's table as they
+// are used: held as 27 values and picked by compares they took 244 registers and 62 us a launch of 2312
+// blocks (D3Q27 MRT, FP32), 46 us so without the values behind.
+template <typename T, typename S, int Q, bool FM>
 __global__ __launch_bounds__(WG) void k_link_step(StepArgs<T, S> a, LinkArgs<T> la)
 {
     using VS = VelSet<Q>;
@@ -1694,82 +855,71 @@ __global__ __launch_bounds__(WG) void k_link_step(StepArgs<T, S> a, LinkArgs<T> 
     const int part_u = __builtin_amdgcn_readfirstlane(a.part[b]);
     const int onb_u = __builtin_amdgcn_readfirstlane(a.onb[b]);
     const int rank = __builtin_amdgcn_readfirstlane(la.onb_solid[b]);
+    const int mask = a.cells_mask[cell];
+    const bool linked = rank >= 0 && mask == CELL_BOUNDARY;
+    const long long cb = (long long)rank * 64 + t;
+    float xq[Q];
+#pragma unroll
+    for (int q = 1; q < Q; q++) xq[q] = linked ? la.X_b[cb + (long long)q * la.ncb] : -1.0f;
     T f[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) f[q] = ST::dec(a.A[(long long)q * a.ncm + cell], (T)VS::w(q));
-    const int mask = a.cells_mask[cell];
     const bool inert = part_u == 0 || mask == CELL_SOLID;
     T fs[Q];
     T rho, u, v, w;
     moments<T, Q>(f, rho, u, v, w);
     collide_cell<T, S, Q>(a, f, fs, rho, u, v, w, inert);
 
-    int nbs[27];
-#pragma unroll
-    for (int s = 0; s < 27; s++) nbs[s] = __builtin_amdgcn_readlane(my_nb, s);
-    const int I = t & 3, J = (t >> 2) & 3, K = t >> 4;
-    // Block of the cell x + c_q (slot table) and of x - c_q.
-    auto slot_of = [&](int dx, int dy, int dz) {
-        const int Ip = I + dx, Jp = J + dy, Kp = K + dz;
-        return (Ip < 0 ? 0 : (Ip >= 4 ? 2 : 1)) + 3 * (Jp < 0 ? 0 : (Jp >= 4 ? 2 : 1)) + 9 * (Kp < 0 ? 0 : (Kp >= 4 ? 2 : 1));
-    };
-    auto cell_of = [&](int dx, int dy, int dz) { return ((I + dx) & 3) + 4 * ((J + dy) & 3) + 16 * ((K + dz) & 3); };
-    auto block_at = [&](int sl) {
-        int r = nbs[0];
-#pragma unroll
-        for (int k = 1; k < 27; k++)
-            if (sl == k) r = nbs[k];
-        return r;
-    };
-
-    const bool linked = rank >= 0 && mask == CELL_BOUNDARY;
-    const long long cb = (long long)rank * 64 + t;
-    float xq[Q];
-#pragma unroll
-    for (int q = 0; q < Q; q++) xq[q] = (linked && q > 0) ? la.X_b[cb + (long long)q * la.ncb] : -1.0f;
-    const bool curved = la.bc_type == 1 && linked;
-    const bool mea2 = la.mea && la.order != 1 && linked;
+    const SlotOf<Q> slot(t);
+    // Block of the cell x + c_q (every lane takes part).
+    auto nb_of = [&](int q) { return __builtin_amdgcn_ds_bpermute(slot(q), my_nb); };
+    const bool curved = FM && la.bc_type == 1 && linked;
 
     // f*_q(x - c_q): within the block from lane (I,J,K) - c_q (every lane takes part), else recomputed.
-    T fm[Q];
-    unsigned long long need = 0;  // bit q: needed and across a block face
-    fm[0] = (T)0;
+    T fm[FM ? Q : 1];
+    unsigned missing = 0;  // bit q: the block behind is missing
+    if constexpr (FM) {
+        const int I = t & 3, J = (t >> 2) & 3, K = t >> 4;
+        const bool mea2 = la.mea && la.order != 1 && linked;
+        unsigned need = 0;  // bit q: needed and across a block face
+        fm[0] = (T)0;
 #pragma unroll
-    for (int q = 1; q < Q; q++) {
-        const int cx = VS::cx(q), cy = VS::cy(q), cz = VS::cz(q);
-        const int src = cell_of(-cx, -cy, -cz);
-        if constexpr (sizeof(T) == 8) {
-            const long long bits = __builtin_bit_cast(long long, fs[q]);
-            const int lo = __shfl((int)(bits & 0xffffffffLL), src, 64), hi = __shfl((int)(bits >> 32), src, 64);
-            fm[q] = __builtin_bit_cast(T, ((long long)hi << 32) | (unsigned)lo);
-        } else {
-            fm[q] = __shfl(fs[q], src, 64);
-        }
-        const bool inside = (unsigned)(I - cx) < 4u && (unsigned)(J - cy) < 4u && (unsigned)(K - cz) < 4u;
-        const bool want = (curved && xq[q] > 0 && xq[q] < 0.5f) || (mea2 && xq[q] > 0);
-        if (want && !inside) need |= 1ull << q;
-    }
-    unsigned long long missing = 0;  // bit q: the block behind is missing
-    while (need) {
-        const int q = __builtin_ctzll(need);
-        need &= need - 1;
-        int cx = 0, cy = 0, cz = 0;
-#pragma unroll
-        for (int p = 1; p < Q; p++)
-            if (p == q) {
-                cx = VS::cx(p);
-                cy = VS::cy(p);
-                cz = VS::cz(p);
+        for (int q = 1; q < Q; q++) {
+            const int cx = VS::cx(q), cy = VS::cy(q), cz = VS::cz(q);
+            const int src = (int)cell_of_link<Q, 0>(t, VS::pb(q));
+            if constexpr (sizeof(T) == 8) {
+                const long long bits = __builtin_bit_cast(long long, fs[q]);
+                const int lo = __shfl((int)(bits & 0xffffffffLL), src, 64), hi = __shfl((int)(bits >> 32), src, 64);
+                fm[q] = __builtin_bit_cast(T, ((long long)hi << 32) | (unsigned)lo);
+            } else {
+                fm[q] = __shfl(fs[q], src, 64);
             }
-        const int nbk = block_at(slot_of(-cx, -cy, -cz));
-        T val = (T)0;
-        if (nbk >= 0)
-            val = post_collision_at<T, S, Q>(a, nbk, cell_of(-cx, -cy, -cz), q);
-        else
-            missing |= 1ull << q;
+            const bool inside = (unsigned)(I - cx) < 4u && (unsigned)(J - cy) < 4u && (unsigned)(K - cz) < 4u;
+            const bool want = (curved && xq[q] > 0 && xq[q] < 0.5f) || (mea2 && xq[q] > 0);
+            if (want && !inside) need |= 1u << q;
+        }
+        while (need) {
+            const int q = __builtin_ctz(need);
+            need &= need - 1;
+            int cx = 0, cy = 0, cz = 0;
 #pragma unroll
-        for (int p = 1; p < Q; p++)
-            if (p == q) fm[p] = val;
+            for (int p = 1; p < Q; p++)
+                if (p == q) {
+                    cx = VS::cx(p);
+                    cy = VS::cy(p);
+                    cz = VS::cz(p);
+                }
+            const int Ip = I - cx + 4, Jp = J - cy + 4, Kp = K - cz + 4;
+            const int nbk = a.nbr_slot[(long long)b * 27 + (Ip >> 2) + 3 * (Jp >> 2) + 9 * (Kp >> 2)];
+            T val = (T)0;
+            if (nbk >= 0)
+                val = post_collision_at<T, S, Q>(a, nbk, (Ip & 3) + 4 * (Jp & 3) + 16 * (Kp & 3), q);
+            else
+                missing |= 1u << q;
+#pragma unroll
+            for (int p = 1; p < Q; p++)
+                if (p == q) fm[p] = val;
+        }
     }
 
     // Momentum exchange before the boundary rules (post_step 0).
@@ -1780,8 +930,9 @@ __global__ __launch_bounds__(WG) void k_link_step(StepArgs<T, S> a, LinkArgs<T> 
             for (int p = 1; p < Q; p++) {
                 if (!VS::half(p)) continue;
                 const int pb = VS::pb(p);
-                if (xq[p] > 0) mea_add<T>(acc, la.order, fs[p], fm[p], xq[p], VS::cx(p), VS::cy(p), VS::cz(p));
-                if (xq[pb] > 0) mea_add<T>(acc, la.order, fs[pb], fm[pb], xq[pb], VS::cx(pb), VS::cy(pb), VS::cz(pb));
+                if (xq[p] > 0) mea_add<T>(acc, FM ? la.order : 1, fs[p], FM ? fm[p] : (T)0, xq[p], VS::cx(p), VS::cy(p), VS::cz(p));
+                if (xq[pb] > 0)
+                    mea_add<T>(acc, FM ? la.order : 1, fs[pb], FM ? fm[pb] : (T)0, xq[pb], VS::cx(pb), VS::cy(pb), VS::cz(pb));
             }
         }
 #pragma unroll
@@ -1791,43 +942,39 @@ __global__ __launch_bounds__(WG) void k_link_step(StepArgs<T, S> a, LinkArgs<T> 
         }
     }
 
-    // Targets of the pushes (blocks in direction +c_q).
-    int nbq[Q];
-#pragma unroll
-    for (int q = 1; q < Q; q++) nbq[q] = block_at(slot_of(VS::cx(q), VS::cy(q), VS::cz(q)));
-    nbq[0] = b;
-
     // Cu_ImposeBC: face hooks and the interpolated bounce-back, pair by pair.
     const bool onb = onb_u == 1 && mask != CELL_SOLID;
-    if (onb) {
+    if (onb_u == 1) {
 #pragma unroll
         for (int p = 1; p < Q; p++) {
             if (!VS::half(p)) continue;
             const int pb = VS::pb(p);
+            const int nbp = nb_of(p), nbb = nb_of(pb);
             T f_p = fs[p], f_q = fs[pb];
-            if (nbq[p] < 0 && nbq[p] != N_SKIPID)
-                f_p = bc_hook<T>(a.bc_preset, a.U, nbq[p], f_p, u, v, w, (T)VS::w(p), (T)VS::cx(p), (T)VS::cy(p), (T)VS::cz(p));
-            if (curved) {
-                const T dQ = (T)xq[p];
-                if (xq[p] > 0 && xq[p] < 0.5f) {
-                    if (!((missing >> p) & 1)) f_p = (T)(2.0) * dQ * f_p + ((T)(1.0) - (T)(2.0) * dQ) * fm[p];
-                } else if (xq[p] >= 0.5f) {
-                    f_p = ((T)(1.0) / ((T)(2.0) * dQ)) * f_p + (((T)(2.0) * dQ - (T)(1.0)) / ((T)(2.0) * dQ)) * f_q;
+            if (nbp < 0 && nbp != N_SKIPID)
+                f_p = bc_hook<T>(a.bc_preset, a.U, nbp, f_p, u, v, w, (T)VS::w(p), (T)VS::cx(p), (T)VS::cy(p), (T)VS::cz(p));
+            if constexpr (FM)
+                if (curved) {
+                    const T dQ = (T)xq[p];
+                    if (xq[p] > 0 && xq[p] < 0.5f) {
+                        if (!((missing >> p) & 1)) f_p = (T)(2.0) * dQ * f_p + ((T)(1.0) - (T)(2.0) * dQ) * fm[p];
+                    } else if (xq[p] >= 0.5f) {
+                        f_p = ((T)(1.0) / ((T)(2.0) * dQ)) * f_p + (((T)(2.0) * dQ - (T)(1.0)) / ((T)(2.0) * dQ)) * f_q;
+                    }
                 }
-            }
-            if (nbq[pb] < 0 && nbq[pb] != N_SKIPID)
-                f_q = bc_hook<T>(a.bc_preset, a.U, nbq[pb], f_q, u, v, w, (T)VS::w(pb), (T)VS::cx(pb), (T)VS::cy(pb),
-                                 (T)VS::cz(pb));
-            if (curved) {
-                const T dQ = (T)xq[pb];
-                if (xq[pb] > 0 && xq[pb] < 0.5f) {
-                    if (!((missing >> pb) & 1)) f_q = (T)(2.0) * dQ * f_q + ((T)(1.0) - (T)(2.0) * dQ) * fm[pb];
-                } else if (xq[pb] >= 0.5f) {
-                    f_q = ((T)(1.0) / ((T)(2.0) * dQ)) * f_q + (((T)(2.0) * dQ - (T)(1.0)) / ((T)(2.0) * dQ)) * f_p;
+            if (nbb < 0 && nbb != N_SKIPID)
+                f_q = bc_hook<T>(a.bc_preset, a.U, nbb, f_q, u, v, w, (T)VS::w(pb), (T)VS::cx(pb), (T)VS::cy(pb), (T)VS::cz(pb));
+            if constexpr (FM)
+                if (curved) {
+                    const T dQ = (T)xq[pb];
+                    if (xq[pb] > 0 && xq[pb] < 0.5f) {
+                        if (!((missing >> pb) & 1)) f_q = (T)(2.0) * dQ * f_q + ((T)(1.0) - (T)(2.0) * dQ) * fm[pb];
+                    } else if (xq[pb] >= 0.5f) {
+                        f_q = ((T)(1.0) / ((T)(2.0) * dQ)) * f_q + (((T)(2.0) * dQ - (T)(1.0)) / ((T)(2.0) * dQ)) * f_p;
+                    }
                 }
-            }
-            fs[p] = f_p;
-            fs[pb] = f_q;
+            fs[p] = onb ? f_p : fs[p];
+            fs[pb] = onb ? f_q : fs[pb];
         }
     }
 
@@ -1835,8 +982,8 @@ __global__ __launch_bounds__(WG) void k_link_step(StepArgs<T, S> a, LinkArgs<T> 
     store_pop(a.B, cell, ST::enc(fs[0], (T)VS::w(0)));
 #pragma unroll
     for (int q = 1; q < Q; q++) {
-        const int nbk = nbq[q];
-        const long long tgt = (long long)nbk * 64 + cell_of(VS::cx(q), VS::cy(q), VS::cz(q));
+        const int nbk = nb_of(q);
+        const long long tgt = (long long)nbk * 64 + cell_of_link<Q, 0>(t, q);
         push_link<T, S, Q>(a, q, fs[q], nbk, tgt, (long long)cell, inert, false, false, u, v, w);
     }
 }
@@ -2011,9 +1158,6 @@ __global__ __launch_bounds__(WG) void k_cv_force(const int *__restrict__ ids, in
 // ---------------------------------------------------------------------------------------------
 // Launchers.
 // ---------------------------------------------------------------------------------------------
-template <typename T>
-static T *Fbuf(Ctx *c, int k) { return static_cast<T *>(c->F[k]); }
-
 static inline int nwg(long long nblocks, int cells) { return (int)((nblocks * cells + WG - 1) / WG); }
 
 template <int Q>
@@ -2053,58 +1197,6 @@ static int refresh_t(Ctx *c, int L)
     return AGAL_OK;
 }
 
-// Fused-step arguments of level L reading population buffer rd (writing rd ^ 1).
-template <typename T, typename S, int Q>
-static StepArgs<T, S> step_args(Ctx *c, int L, int rd, int vmode = 0)
-{
-    StepArgs<T, S> a;
-    a.ids = c->order_L(L);  // the level's blocks in traversal order
-    a.n = c->n_ids[L];
-    a.A = Fbuf<S>(c, rd);
-    a.B = Fbuf<S>(c, rd ^ 1);
-    a.ncm = c->n_maxcells;
-    a.nbr_slot = c->nbr_slot;
-    a.part = c->part;
-    a.simple = c->simple;
-    a.cells_mask = c->cells_mask;
-    a.onb = c->onb;
-    const T dx_L = (T)c->dxf_vec[L], tau_L = (T)c->tau_vec[L];
-    a.omeg = dx_L / tau_L;
-    a.omegp = (T)(1.0) - a.omeg;
-    a.mrt = c->P.collision == AGAL_MRT;
-    {
-        const double s[6] = {c->P.s1, c->P.s2, c->P.s3, c->P.s4, c->P.s5, c->P.s6};
-        for (int k = 0; k < 27; k++) a.ck[k] = (T)0;
-        for (int k = 0; k < Q; k++) {
-            const int rc = Mrt<Q>::rate(k);
-            if (rc == 0) continue;
-            const T rate = rc == 1 ? a.omeg : (T)s[rc - 2];
-            a.ck[k] = (T)((double)rate / (double)mrt_norm<Q>(k));
-        }
-    }
-    a.U = (T)c->P.bc_velocity;
-    a.bc_preset = c->P.bc_preset;
-    // Each level has its own exception list: levels share launches.
-    a.exc_idx = c->exc_idx + (size_t)3 * c->exc_cap * L;
-    a.exc_val = static_cast<T *>(c->exc_val) + (size_t)c->exc_cap * L;
-    a.exc_count = c->exc_count + 2 * L;
-    a.exc_cap = c->exc_cap;
-    const int XL = c->MAX_LEVELS;  // the extra list's slot
-    a.vmode = vmode;
-    a.flags = c->simple;
-    a.va_idx = c->exc_idx + (size_t)3 * c->exc_cap * XL;
-    a.va_val = static_cast<T *>(c->exc_val) + (size_t)c->exc_cap * XL;
-    a.va_count = c->exc_count + 2 * XL;
-    a.x_head = c->exc_head;
-    a.x_next = c->exc_next;
-    if (vmode == 1) {
-        a.exc_idx = c->exc_idx + (size_t)3 * c->exc_cap * XL;
-        a.exc_val = static_cast<T *>(c->exc_val) + (size_t)c->exc_cap * XL;
-        a.exc_count = c->exc_count + 2 * XL;
-    }
-    return a;
-}
-
 // The extra-list mode of level L in the fused launch being issued: only for the finest level of a
 // 3D set inside a coarse step.
 template <int Q>
@@ -2112,7 +1204,8 @@ static int pair_mode(const Ctx *c, int L)
 {
     // Linked blocks recompute neighbours' collisions from the input buffer as it is stored, so
     // with links every sub-step resolves its exceptions by a fixup instead.
-    return (VelSet<Q>::DIM == 3 && c->defer_coarse && L == c->MAX_LEVELS - 1 && !c->links_on) ? c->fine_pair : 0;
+    if (VelSet<Q>::DIM != 3 || !c->defer_coarse || L != c->MAX_LEVELS - 1 || c->links_on) return 0;
+    return c->fine_pair == 1 && inplace_ok(c, L) ? VMODE_EVEN : c->fine_pair;
 }
 
 // The momentum-exchange force (force type 0) is evaluated on the finest level's last sub-step of a
@@ -2123,6 +1216,11 @@ static bool mea_due(const Ctx *c, int L)
     if (!mea_active(c) || L != c->MAX_LEVELS - 1) return false;
     const bool multi = c->MAX_LEVELS > 1 && c->MAX_LEVELS != c->N_LEVEL_START + 1;
     return !multi || c->global_Liter == (1 << (c->MAX_LEVELS - 1)) - 1;
+}
+
+static bool link_step_due(const Ctx *c, int L)
+{
+    return c->links_on && c->lk_n[L] > 0 && (c->P.S_BC_TYPE == 1 || mea_due(c, L));
 }
 
 template <typename T>
@@ -2144,14 +1242,18 @@ static LinkArgs<T> link_args(Ctx *c, int L, bool mea)
     return la;
 }
 
-// The linked blocks' sub-step of level L reading buffer rd, on stream s.
+// The linked blocks' sub-step of level L reading buffer rd, on stream s, where it differs from that of
+// other blocks: with the interpolated bounce-back, or when the momentum exchange is due.  Otherwise the
+// fused step takes the linked blocks like any (link_step_due).
 template <typename T, typename S, int Q>
 static int launch_link_step(Ctx *c, int L, int rd, hipStream_t s)
 {
     if constexpr (VelSet<Q>::DIM == 3) {
-        if (!c->links_on || c->lk_n[L] <= 0) return AGAL_OK;
+        if (!link_step_due(c, L)) return AGAL_OK;
         const LinkArgs<T> la = link_args<T>(c, L, mea_due(c, L));
-        hipLaunchKernelGGL((k_link_step<T, S, Q>), dim3((unsigned)((la.n + WG / 64 - 1) / (WG / 64))), dim3(WG), 0, s,
+        const bool fm = la.bc_type == 1 || (la.mea && la.order != 1);
+        hipLaunchKernelGGL((fm ? k_link_step<T, S, Q, true> : k_link_step<T, S, Q, false>),
+                           dim3((unsigned)((la.n + WG / 64 - 1) / (WG / 64))), dim3(WG), 0, s,
                            step_args<T, S, Q>(c, L, rd, 0), la);
         AGAL_HIP(c, hipGetLastError());
     }
@@ -2175,57 +1277,12 @@ static InterpArgs<T, S> interp_args(Ctx *c, int L, const int *ids, int n, T rati
     return ia;
 }
 
-// Exception lists waiting for their fixup: up to MAXLV of the pending levels in `mask` go into fa
-// (with the buffer that the launch which left the list wrote) and leave the pending set.
-template <typename T, typename S>
-static int take_fixups(Ctx *c, unsigned mask, FixupArgs<T, S> &fa, unsigned &wmask)
-{
-    int n = 0;
-    std::vector<std::pair<int, int>> keep;
-    for (const auto &pf : c->pending_fix) {
-        const int L = pf.first, buf = pf.second;
-        if (!((mask >> L) & 1) || n == MAXLV) {
-            keep.push_back(pf);
-            continue;
-        }
-        fa.B[n] = Fbuf<S>(c, buf);
-        fa.exc_idx[n] = c->exc_idx + (size_t)3 * c->exc_cap * L;
-        fa.exc_val[n] = static_cast<T *>(c->exc_val) + (size_t)c->exc_cap * L;
-        fa.exc_count[n] = c->exc_count + 2 * L;
-        fa.va_count[n] = L == c->MAX_LEVELS - 1 ? c->exc_count + 2 * c->MAX_LEVELS : nullptr;
-        wmask |= res_bit(L, buf);
-        n++;
-    }
-    c->pending_fix = keep;
-    fa.ncm = c->n_maxcells;
-    fa.exc_cap = c->exc_cap;
-    return n;
-}
-
-// Fixup launches for the pending levels in `mask`.
-template <typename T, typename S, int Q>
-static int launch_fixups(Ctx *c, unsigned mask)
-{
-    for (;;) {
-        FixupArgs<T, S> fa;
-        unsigned wmask = 0;
-        const int n = take_fixups<T, S>(c, mask, fa, wmask);
-        if (n == 0) return AGAL_OK;
-        hipStream_t s = sched_begin(c, 0, 0, wmask);
-        hipLaunchKernelGGL((k_fixup<T, S, Q>), dim3(n), dim3(WG), 0, s, fa);
-        AGAL_HIP(c, hipGetLastError());
-        int st = sched_done(c, s, 0, 0, wmask);
-        if (st) return st;
-    }
-}
-
 // Fused step of levels[j] reading buffers rd[j], up to MAXLV levels per launch.  With `ia`, the
 // first launch also interpolates level interp_L's interface parents (reading the buffer those
-// sub-steps read).  Exception lists: inside a coarse step (defer_coarse) a launch leaves its
-// levels' lists pending; pending lists of levels the launch touches are resolved by a fixup
-// launch before it, the others by workgroups of the launch itself.  Outside a coarse step the
-// fixup follows at once.  A coarse level alone goes to its level stream (the recorded step's
-// scheduler); launches that hold the finest level stay on the context stream.
+// sub-steps read).  Exception lists: those pending are resolved first (fold_fixups); the launch leaves
+// its own levels' pending; outside a coarse step (defer_coarse) a fixup launch follows at once.  A coarse
+// level alone goes to its level stream (the recorded step's scheduler); launches that hold the finest
+// level stay on the context stream.
 template <typename T, typename S, int Q>
 static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const InterpArgs<T, S> *ia = nullptr,
                         int interp_L = -1)
@@ -2234,8 +1291,7 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
     int st;
     unsigned touch = 0;
     for (int j = 0; j < nl; j++) touch |= 1u << levels[j];
-    if (ia) touch |= (1u << interp_L) | (1u << (interp_L + 1));
-    if ((st = launch_fixups<T, S, Q>(c, touch))) return st;
+    if (ia) touch |= 3u << interp_L;
     for (int base = 0; base < nl || (base == 0 && ia); base += MAXLV) {
         MultiStep<T, S> m;
         StepExtras<T, S> x;
@@ -2247,12 +1303,14 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
         int first = -1;
         for (int j = base; j < nl && j < base + MAXLV; j++) {
             const int L = levels[j], n = c->n_ids[L];
+            const int mode = pair_mode<Q>(c, L);
             rmask |= res_bit(L, rd[j]);
-            wmask |= res_bit(L, rd[j] ^ 1);
+            wmask |= res_bit(L, mode == VMODE_EVEN ? rd[j] : rd[j] ^ 1);
             if (n <= 0) continue;
             finest = finest || L == c->MAX_LEVELS - 1;
             if (first < 0) first = L;
-            m.lv[m.nlv] = step_args<T, S, Q>(c, L, rd[j], pair_mode<Q>(c, L));
+            m.lv[m.nlv] = step_args<T, S, Q>(c, L, rd[j], mode);
+            m.lv[m.nlv].skip_linked = link_step_due(c, L);
             m.start[m.nlv] = (int)waves;
             waves += (n + BPW - 1) / BPW;
             cells += (double)n * CELLS;
@@ -2261,7 +1319,6 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
         for (int k = m.nlv; k <= MAXLV; k++) m.start[k] = (int)waves;
         x.step_wgs = m.nlv ? (int)((waves + WG / 64 - 1) / (WG / 64) + 7) / 8 * 8 : 0;  // a multiple of the XCD count
         x.interp_wgs = 0;
-        x.fix_wgs = 0;
         if (base == 0) {
             if (ia && ia->n > 0) {
                 x.ia = *ia;
@@ -2269,40 +1326,35 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
                 rmask |= res_bit(interp_L, rd[0]);
                 wmask |= res_bit(interp_L + 1, c->cur[interp_L + 1]);
             }
-            if (c->defer_coarse && !c->timing.enabled) x.fix_wgs = take_fixups<T, S>(c, ~touch, x.fa, wmask);
         }
-        x.lead = (x.interp_wgs + x.fix_wgs + 7) / 8 * 8;
-        if (x.step_wgs + x.interp_wgs + x.fix_wgs == 0) continue;
-        const int slot = (finest || m.nlv != 1 || x.interp_wgs || x.fix_wgs) ? 0 : 1 + first;
-        hipStream_t s = sched_begin(c, slot, rmask, wmask);
+        x.lead = (x.interp_wgs + 7) / 8 * 8;
+        if (x.step_wgs + x.interp_wgs == 0) continue;
         const int grid = x.lead + x.step_wgs;
-        // The matrix-core MRT variant: FP32 compute, 3D sets of 19 / 27 directions, when enabled.
-        constexpr bool MF_OK = sizeof(T) == 4 && (Q == 19 || Q == 27);
-        const bool mf = MF_OK && c->P.collision == AGAL_MRT && c->mrt_mfma;
-        auto kern = mf ? (void (*)(MultiStep<T, S>, StepExtras<T, S>))k_collide_stream<T, S, Q, MF_OK>
-                       : (void (*)(MultiStep<T, S>, StepExtras<T, S>))k_collide_stream<T, S, Q, false>;
-        if (c->timing.enabled && m.nlv) {
-            // Events recorded by the dispatch itself: they bracket the kernel's execution.
-            hipEvent_t e0 = nullptr, e1 = nullptr;
-            AGAL_HIP(c, hipEventCreate(&e0));
-            AGAL_HIP(c, hipEventCreate(&e1));
-            hipExtLaunchKernelGGL(kern, dim3(grid), dim3(WG), 0, s, e0, e1, 0, m, x);
-            AGAL_HIP(c, hipGetLastError());
-            c->timing.ev_pairs.push_back(e0);
-            c->timing.ev_pairs.push_back(e1);
-            c->timing.fused_launches++;
-            c->timing.fused_cells += cells;
-        } else {
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(WG), 0, s, m, x);
-            AGAL_HIP(c, hipGetLastError());
-        }
+        if ((st = fold_fixups<T, S, Q>(c, grid, touch, x.fa, wmask))) return st;
+        const int slot = (finest || m.nlv != 1 || x.interp_wgs || x.fa.n) ? 0 : 1 + first;
+        hipStream_t s = sched_begin(c, slot, rmask, wmask);
+        // One kernel per collision operator: BGK alone needs fewer registers than MRT's moments.  The
+        // matrix-core MRT variant: FP32 compute, 3D sets, when enabled.
+        using K = void (*)(MultiStep<T, S>, StepExtras<T, S>);
+        const bool mrt = c->P.collision == AGAL_MRT, fold = x.fa.n > 0;
+        K kern = mrt ? (fold ? (K)k_collide_stream<T, S, Q, COLL_MRT, true> : (K)k_collide_stream<T, S, Q, COLL_MRT, false>)
+                     : (fold ? (K)k_collide_stream<T, S, Q, COLL_BGK, true> : (K)k_collide_stream<T, S, Q, COLL_BGK, false>);
+        if constexpr (sizeof(T) == 4 && VelSet<Q>::DIM == 3)
+            if (mrt && c->mrt_mfma)
+                kern = fold ? (K)k_collide_stream<T, S, Q, COLL_MFMA, true> : (K)k_collide_stream<T, S, Q, COLL_MFMA, false>;
+        if ((st = launch_timed(c, kern, grid, s, cells, m, x))) return st;
         for (int j = base; j < nl && j < base + MAXLV; j++)
             if ((st = launch_link_step<T, S, Q>(c, levels[j], rd[j], s))) return st;
         if ((st = sched_done(c, s, slot, rmask, wmask))) return st;
         // A list left for the next finest sub-step (pair mode 1) is not pending a fixup.
-        for (int j = base; j < nl && j < base + MAXLV; j++)
-            if (pair_mode<Q>(c, levels[j]) != 1) c->pending_fix.push_back({levels[j], rd[j] ^ 1});
-        if (!c->defer_coarse && (st = launch_fixups<T, S, Q>(c, ~0u))) return st;
+        for (int j = base; j < nl && j < base + MAXLV; j++) {
+            const int mode = pair_mode<Q>(c, levels[j]);
+            if (mode == VMODE_EVEN)
+                c->leave_pending(levels[j], rd[j], 1);
+            else if (mode != 1)
+                c->leave_pending(levels[j], rd[j] ^ 1, 0);
+        }
+        if (!c->defer_coarse && (st = launch_fixups<T, S, Q>(c))) return st;
     }
     return AGAL_OK;
 }
@@ -2320,7 +1372,10 @@ static int collide_stream_t(Ctx *c, int L)
         return AGAL_OK;
     }
     std::vector<int> lv{L}, rd{c->cur[L]};
-    c->cur[L] ^= 1;
+    // An in-place pair leaves the level in the buffer that it read.
+    const bool even = pair_mode<Q>(c, L) == VMODE_EVEN;
+    if (!even && c->fine_pair == 2 && c->defer_coarse && inplace_ok(c, L)) return launch_odd_step(c, L);
+    if (!even) c->cur[L] ^= 1;
     for (const auto &d : c->deferred) {
         lv.push_back(d.first);
         rd.push_back(d.second);
@@ -2340,7 +1395,6 @@ static int interp_collide_t(Ctx *c, int L)
     // The timed pass (timing.enabled) keeps the interpolation apart, so that the events around a
     // fused launch time the fused step alone.
     if (!c->defer_coarse || c->timing.enabled || c->P.interp_order == AGAL_INTERP_CUBIC || L >= c->MAX_LEVELS - 1) {
-        if ((st = launch_fixups<T, S, Q>(c, (1u << L) | (2u << L)))) return st;  // levels L, L+1
         if ((st = launch_interpolate(c, L, AGAL_INTERP_INTERFACE))) return st;
         return launch_collide_stream(c, L);
     }
@@ -2370,13 +1424,7 @@ static int flush_deferred_t(Ctx *c)
         c->deferred.clear();
         if ((st = launch_fused<T, S, Q>(c, lv.data(), rd.data(), (int)lv.size()))) return st;
     }
-    return launch_fixups<T, S, Q>(c, ~0u);
-}
-
-template <typename T, typename S, int Q>
-static int fix_pending_t(Ctx *c)
-{
-    return launch_fixups<T, S, Q>(c, ~0u);
+    return launch_fixups<T, S, Q>(c);
 }
 
 template <typename T, typename S, int Q>
@@ -2394,6 +1442,7 @@ static int interpolate_t(Ctx *c, int L, int var)
         n = c->n_ids[L];
     }
     if (n <= 0) return AGAL_OK;
+    if (int st = launch_fixups_for<T, S, Q>(c, 3u << L)) return st;
     const unsigned rl = res_bit(L, c->cur[L]), wl = res_bit(L + 1, c->cur[L + 1]);
     hipStream_t s = sched_begin(c, 0, rl, wl);
     if (c->P.interp_order == AGAL_INTERP_CUBIC) {
@@ -2428,10 +1477,13 @@ static int average_t(Ctx *c, int L, int var)
         n = c->n_ids[L];
     }
     if (n <= 0) return AGAL_OK;
-    const unsigned rl = res_bit(L + 1, c->cur[L + 1]), wl = res_bit(L, c->cur[L]);
+    const unsigned rl = res_bit(L + 1, c->cur[L + 1]);
+    unsigned wl = res_bit(L, c->cur[L]);
+    FixupArgs<T, S> fa;
+    const int grid = nwg(n, VelSet<Q>::CELLS / 2 * (VelSet<Q>::DIM == 3 ? 8 : 4));
+    if (int st = fold_fixups<T, S, Q>(c, grid, 3u << L, fa, wl)) return st;
     hipStream_t s = sched_begin(c, 0, rl, wl);
-    hipLaunchKernelGGL((k_average<T, S, Q>), dim3(nwg(n, VelSet<Q>::CELLS / 2 * (VelSet<Q>::DIM == 3 ? 8 : 4))), dim3(WG),
-                       0, s, ids, n, Fbuf<S>(c, c->cur[L]), Fbuf<S>(c, c->cur[L + 1]), c->n_maxcells, c->nbr_child,
+    hipLaunchKernelGGL((fa.n ? k_average<T, S, Q, true> : k_average<T, S, Q, false>), dim3(grid), dim3(WG), 0, s, fa, ids, n, Fbuf<S>(c, c->cur[L]), Fbuf<S>(c, c->cur[L + 1]), c->n_maxcells, c->nbr_child,
                        c->blk_mask, c->cells_mask, var, ratio);
     AGAL_HIP(c, hipGetLastError());
     return sched_done(c, s, 0, rl, wl);
@@ -2449,31 +1501,16 @@ static int avg_interp_t(Ctx *c, int L)
     if (n <= 0) return AGAL_OK;
     const T ratio_avg = (T)c->tau_vec[L] / (T)c->tau_vec[L + 1];
     const T ratio_int = (T)c->tau_vec[L + 1] / (T)c->tau_vec[L];
-    const unsigned m = res_bit(L, c->cur[L]) | res_bit(L + 1, c->cur[L + 1]);
+    unsigned m = res_bit(L, c->cur[L]) | res_bit(L + 1, c->cur[L + 1]);
+    FixupArgs<T, S> fa;
+    if (int st = fold_fixups<T, S, Q>(c, interp_grid<Q>(n), 3u << L, fa, m)) return st;
     hipStream_t s = sched_begin(c, 0, m, m);
-    hipLaunchKernelGGL((k_avg_interp<T, S, Q>), dim3(interp_grid<Q>(n)), dim3(IWG), 0, s, c->iface_L(L), n,
+    hipLaunchKernelGGL((fa.n ? k_avg_interp<T, S, Q, true> : k_avg_interp<T, S, Q, false>), dim3(interp_grid<Q>(n)), dim3(IWG), 0, s, fa, c->iface_L(L), n,
                        Fbuf<S>(c, c->cur[L]), Fbuf<S>(c, c->cur[L + 1]), c->n_maxcells, c->nbr_child, c->blk_mask,
                        c->cells_mask, ratio_avg, ratio_int);
     AGAL_HIP(c, hipGetLastError());
     return sched_done(c, s, 0, m, m);
 }
-
-#define AGAL_DISPATCH_Q(c, FN, T, S, ...)                                                  \
-    do {                                                                                   \
-        if ((c)->Q == 9) return FN<T, S, 9>(__VA_ARGS__);                                  \
-        if ((c)->Q == 19) return FN<T, S, 19>(__VA_ARGS__);                                \
-        if ((c)->Q == 27) return FN<T, S, 27>(__VA_ARGS__);                                \
-    } while (0)
-#define AGAL_DISPATCH(c, FN, ...)                                                          \
-    do {                                                                                   \
-        switch ((c)->precision) {                                                          \
-            case AGAL_FP64: AGAL_DISPATCH_Q(c, FN, double, double, __VA_ARGS__); break;    \
-            case AGAL_FP32: AGAL_DISPATCH_Q(c, FN, float, float, __VA_ARGS__); break;      \
-            case AGAL_FP16: AGAL_DISPATCH_Q(c, FN, float, _Float16, __VA_ARGS__); break;   \
-            case AGAL_BF16: AGAL_DISPATCH_Q(c, FN, float, bf16s, __VA_ARGS__); break;      \
-        }                                                                                  \
-        return AGAL_ERR_ARG;                                                               \
-    } while (0)
 
 template <typename T, typename S, int Q>
 static int cv_force_t(Ctx *c, int L, int post)
@@ -2523,6 +1560,7 @@ static int mea_post_t(Ctx *c)
     return AGAL_OK;
 }
 
+bool inplace_pair(const Ctx *c, int L) { return inplace_ok(c, L); }
 int launch_mea_post(Ctx *c) { AGAL_DISPATCH(c, mea_post_t, c); }
 int launch_cv_force(Ctx *c, int L, int post) { AGAL_DISPATCH(c, cv_force_t, c, L, post); }
 int launch_set_ic(Ctx *c, int L) { AGAL_DISPATCH(c, set_ic_t, c, L); }
@@ -2530,7 +1568,6 @@ int launch_refresh(Ctx *c, int L) { AGAL_DISPATCH(c, refresh_t, c, L); }
 int launch_collide_stream(Ctx *c, int L) { AGAL_DISPATCH(c, collide_stream_t, c, L); }
 int launch_flush_deferred(Ctx *c) { AGAL_DISPATCH(c, flush_deferred_t, c); }
 int launch_interp_collide(Ctx *c, int L) { AGAL_DISPATCH(c, interp_collide_t, c, L); }
-int launch_fix_pending(Ctx *c) { AGAL_DISPATCH(c, fix_pending_t, c); }
 int launch_interpolate(Ctx *c, int L, int var) { AGAL_DISPATCH(c, interpolate_t, c, L, var); }
 int launch_average(Ctx *c, int L, int var) { AGAL_DISPATCH(c, average_t, c, L, var); }
 int launch_average_interpolate(Ctx *c, int L) { AGAL_DISPATCH(c, avg_interp_t, c, L); }

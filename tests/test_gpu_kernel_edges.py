@@ -2,6 +2,8 @@
 of their ranges, against the CPU restatement."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -47,3 +49,80 @@ def test_cubic_interpolation_of_other_sets_and_storage(vs, prec):
     assert g.refresh_sizes().n_ids[1] > 0
     bad = compare_states(g.state(), o.state())
     assert not bad, "\n".join(bad)
+
+
+def _perturbed(m, o, seed):
+    """The same populations in both contexts, many of them non-positive."""
+    f = o.populations()
+    f = f * (1.0 + 1.5 * np.random.default_rng(seed).standard_normal(f.shape).astype(f.dtype))
+    m.set_populations(f)
+    o.set_populations(f)
+
+
+@pytest.mark.parametrize("vs,prec,coll", [(capi.D3Q19, capi.FP32, capi.BGK), (capi.D3Q19, capi.FP64, capi.MRT),
+                                          (capi.D3Q27, capi.FP16, capi.MRT), (capi.D3Q27, capi.BF16, capi.BGK)])
+@pytest.mark.parametrize("periodic", [0, 1])
+def test_in_place_pairs_on_one_level(vs, prec, coll, periodic):
+    """One to nine steps in one call (in-place pairs, an odd one out, several recorded graphs) on a root
+    grid of unequal sides, two blocks wide along z, with lid or periodic faces, from populations that
+    fail the swap guard in many links: the exchange before each second sub-step and the fixups after
+    it, bit for bit."""
+    p = ldc_params(vs=vs, N=16, Re=20.0, levels=1, prec=prec, collision=coll)
+    p.L_fy, p.L_fz = 0.75, 0.5
+    p.PERIODIC_X = p.PERIODIC_Z = periodic
+    g, o = LbmMesh(p, 1024), OracleMesh(p, 1024)  # lists of 65 536 entries
+    for m in (g, o):
+        m.S_SetIC(0)
+    _perturbed(g, o, 11)
+    i = 0
+    for n in (1, 2, 3, 4, 9):
+        for m in (g, o):
+            m.advance_loop(i, n)
+        i += n
+        bad = compare_states(g.state(), o.state())
+        assert not bad, f"after {n}: " + "\n".join(bad)
+    g.close()
+
+
+def test_pairs_leave_a_level_with_solid_cells_to_the_general_path():
+    """A cell turned solid makes its neighbourhood general: the level's sub-steps then run one by one,
+    and again in place once the cell is fluid."""
+    p = ldc_params(vs=capi.D3Q19, N=16, Re=20.0, levels=1, prec=capi.FP32)
+    g, o = LbmMesh(p, 128), OracleMesh(p, 128)
+    for m in (g, o):
+        m.S_SetIC(0)
+        m.advance_loop(0, 4)
+    mask = o.cell_masks()
+    for solid in (True, False):
+        mask[64 * 21 + 27] = capi.CELL_SOLID if solid else capi.CELL_INTERIOR
+        nb = g.n_blocks()
+        g._call("upload_cell_masks", capi.np_ptr(np.ascontiguousarray(mask[: 64 * nb]), ctypes.c_int), nb)
+        o.set_cell_masks(mask[: 64 * nb])
+        for m in (g, o):
+            m.advance_loop(4 if solid else 10, 6)
+        bad = compare_states(g.state(), o.state())
+        assert not bad, f"solid {solid}: " + "\n".join(bad)
+    g.close()
+
+
+@pytest.mark.parametrize("vs,prec", [(capi.D2Q9, capi.FP32), (capi.D3Q19, capi.FP32)])
+def test_pending_lists_resolved_by_the_next_kernel(vs, prec):
+    """Guard failures on every level of a refined mesh: each kernel of the coarse step (fused step,
+    in-place second sub-step, average, average + interpolation) finds lists to resolve, with several
+    workgroups waiting for the one that does."""
+    p = ldc_params(vs=vs, N=32 if vs == capi.D2Q9 else 16, Re=40.0, levels=3, P_REFINE=1 << 28, prec=prec)
+    g, o = LbmMesh(p, 4096), OracleMesh(p, 4096)
+    for m in (g, o):
+        m.S_SetIC(0)
+        for L in range(2):
+            ids = m.id_set(L)
+            m.mark_blocks(ids[m.coords()[0, ids] < 0.3 / (L + 1)], capi.REF_MARK_REFINE)
+            m.M_RefineAndCoarsenBlocks()
+    assert g.refresh_sizes().n_ids[2] > 0
+    _perturbed(g, o, 5)
+    for i in range(3):
+        for m in (g, o):
+            m.advance_loop(2 * i, 2)
+        bad = compare_states(g.state(), o.state())
+        assert not bad, "\n".join(bad)
+    g.close()
