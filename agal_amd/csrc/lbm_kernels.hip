@@ -168,9 +168,47 @@ struct InterpLds {  // LDS of one interpolation workgroup
     static constexpr int ALL = Q * PPW * CELLS, COEF = PPW * Q * NCH * InterpCoef<T, Q>::N;
 };
 
+// The ghost cells of a 3D parent's children (512 cells, of which an interface block typically has 128),
+// listed in LDS, so that the interpolation's lanes take one ghost cell each instead of two cells each
+// that may or may not be one.  The workgroup's four wavefronts call ghost_masks before, ghost_list after
+// one barrier, and read the list after another.
+struct GhostList {
+    unsigned long long mask[8];  // per child
+    unsigned short cell[512];    // child * 64 + cell, `total` of them
+};
+
+__device__ __forceinline__ void ghost_masks(GhostList &g, const int *__restrict__ cells_mask, int fc, bool work)
+{
+    const int c = threadIdx.x >> 6, t = threadIdx.x & 63;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const bool put = work && cells_mask[(long long)(fc + c + 4 * h) * 64 + t] == CELL_GHOST;
+        const unsigned long long m = __ballot(put);
+        if (t == 0) g.mask[c + 4 * h] = m;
+    }
+}
+
+__device__ __forceinline__ int ghost_list(GhostList &g)
+{
+    const int c = threadIdx.x >> 6, t = threadIdx.x & 63;
+    int total = 0, off[2] = {0, 0};
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        if (k == c) off[0] = total;
+        if (k == c + 4) off[1] = total;
+        total += __popcll(g.mask[k]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const unsigned long long m = g.mask[c + 4 * h];
+        if ((m >> t) & 1) g.cell[off[h] + __popcll(m & ((1ull << t) - 1))] = (unsigned short)((c + 4 * h) * 64 + t);
+    }
+    return total;
+}
+
 // Workgroup `wg` of the interpolation (IWG threads): its parents, their children's cells.
 template <typename T, typename S, int Q, bool ADDED>
-__device__ __forceinline__ void interp_parents(const InterpArgs<T, S> &ia, int wg, T *s_all, T *s_coef)
+__device__ __forceinline__ void interp_parents(const InterpArgs<T, S> &ia, int wg, T *s_all, T *s_coef, GhostList &s_ghost)
 {
     using VS = VelSet<Q>;
     constexpr int CELLS = VS::CELLS, NCH = VS::CHILDREN, HALF = NCH / 2;
@@ -190,8 +228,11 @@ __device__ __forceinline__ void interp_parents(const InterpArgs<T, S> &ia, int w
         work = fc >= 0 && (ADDED ? (ia.ref[b] == REF_MARK_REFINE) : (ia.blk_mask[b] == BLK_INTERFACE));
     }
     // The children's cell masks, fetched before the barrier.
+    constexpr bool LIST = VS::DIM == 3 && !ADDED;
     bool put[2] = {false, false};
-    if (work)
+    if constexpr (LIST)
+        ghost_masks(s_ghost, ia.cells_mask, fc, work);
+    else if (work)
 #pragma unroll
         for (int h = 0; h < 2; h++)
             put[h] = ADDED || ia.cells_mask[(long long)(fc + c + h * HALF) * CELLS + t] == CELL_GHOST;
@@ -212,9 +253,18 @@ __device__ __forceinline__ void interp_parents(const InterpArgs<T, S> &ia, int w
         }
     }
     __syncthreads();
+    int total = 0;
+    if constexpr (LIST) total = ghost_list(s_ghost);
     interp_coefficients<T, Q, PPW, IWG>(s_all, s_coef);
     __syncthreads();
     if (!work) return;
+    if constexpr (LIST) {
+        for (int k = threadIdx.x; k < total; k += IWG) {
+            const int e = s_ghost.cell[k];
+            interp_child<T, S, Q>(s_coef, e >> 6, e & 63, ia.Fc, ncm, (long long)fc * 64 + e);
+        }
+        return;
+    }
 #pragma unroll
     for (int h = 0; h < 2; h++)
         if (put[h])
@@ -228,7 +278,8 @@ __global__ __launch_bounds__(IWG) void k_interp(InterpArgs<T, S> ia)
     using IL = InterpLds<T, Q>;
     __shared__ T s_all[IL::ALL];
     __shared__ T s_coef[IL::COEF];
-    interp_parents<T, S, Q, ADDED>(ia, blockIdx.x, s_all, s_coef);
+    __shared__ GhostList s_ghost;
+    interp_parents<T, S, Q, ADDED>(ia, blockIdx.x, s_all, s_coef, s_ghost);
 }
 
 // Sum over the NG lanes of each lane group (NG consecutive lanes, NG = 8 in 3D, 4 in 2D) of the
@@ -257,6 +308,59 @@ __device__ __forceinline__ void group_sums(const T *v, T *acc, T *lds)
     }
 }
 
+// Average of one 3D parent block by a workgroup of four wavefronts (Cu_Average, solver_lbm_kernels_comm.cu:
+// 174-347).  Eight consecutive lanes serve one parent cell, each lane loading and rescaling one child
+// cell of its 2x2x2 group; the sum is formed in the reference's order (group_sums) and each lane hands
+// the directions p = lane (mod 8) to put(t, p, value).  Every wavefront finds the parent cells that are
+// averaged (their first child cell is an interface cell; ave_type > 0: is not a ghost) with one load and
+// a ballot and deals them out in eights, so lanes are not spent on the others: an interface block has
+// typically 16 of its 64 cells averaged.  Returns the mask of the averaged cells.
+template <typename T, typename S, int Q, class Put>
+__device__ __forceinline__ unsigned long long average_block_3d(const S *Fc, long long ncm, const int *__restrict__ cells_mask,
+                                                               int fc, int ave_type, T ratio, T *s_red, Put put)
+{
+    using VS = VelSet<Q>;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, k = lane & 7;
+    // First child cell of parent cell t.
+    auto first = [&](int t) {
+        const int I = t & 3, J = (t >> 2) & 3, K = t >> 4;
+        const int c = (I >> 1) + 2 * (J >> 1) + 4 * (K >> 1);
+        return (long long)(fc + c) * 64 + 2 * (I & 1) + 8 * (J & 1) + 32 * (K & 1);
+    };
+    int m = cells_mask[first(lane)];
+    if (ave_type > 0 && m < 2) m = 1;
+    const unsigned long long done = __ballot(m == 1);
+    const int cnt = __popcll(done);
+    // Lane r of `list`: the r-th averaged cell.  (Lanes of the others send beyond them.)
+    const int rank = __popcll(done & ((1ull << lane) - 1));
+    const int list = __builtin_amdgcn_ds_permute(4 * (m == 1 ? rank : cnt + lane - rank), lane);
+    for (int n0 = 8 * wv; n0 < cnt; n0 += 32) {
+        const int r = n0 + (lane >> 3);
+        const int t = __shfl(list, r < cnt ? r : n0, 64);
+        T s[Q];
+        const long long cell = first(t) + (k & 1) + 4 * ((k >> 1) & 1) + 16 * (k >> 2);
+#pragma unroll
+        for (int p = 0; p < Q; p++) s[p] = Store<T, S>::dec(Fc[(long long)p * ncm + cell], (T)VS::w(p));
+        T rho, u, v, w;
+        moments<T, Q>(s, rho, u, v, w);
+        const T udotu = u * u + v * v + w * w;
+#pragma unroll
+        for (int p = 0; p < Q; p++) {
+            T cdotu = cdot<T, Q>(p, u, v, w);
+            T fe = (T)VS::w(p) * rho * ((T)(1.0) + (T)(3.0) * cdotu + (T)(4.5) * cdotu * cdotu - (T)(1.5) * udotu);
+            s[p] = fe + (s[p] - fe) * ratio;
+        }
+        T acc[(Q + 7) / 8];
+        group_sums<T, Q, 8>(s, acc, s_red + wv * Q * 65);
+#pragma unroll
+        for (int j = 0; j < (Q + 7) / 8; j++) {
+            const int p = k + 8 * j;
+            if (r < cnt && p < Q) put(t, p, (T)(0.125) * acc[j]);
+        }
+    }
+    return done;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Fine -> coarse then coarse -> fine in one launch: the pair "average(L) in INTERFACE mode, then
 // linear interpolation(L) in INTERFACE mode" that the advance runs between the two sub-cycles of
@@ -266,6 +370,8 @@ __device__ __forceinline__ void group_sums(const T *v, T *acc, T *lds)
 // writes the children's ghost cells (mask 2).  A workgroup therefore does both for its parents:
 // the averaged values go to the pool and, as the pool will hold them, to LDS, from where the
 // interpolation stage takes them.  Arithmetic and order are those of k_average and k_interp.
+// D3Q19 FP32, 3008 parents: 35 -> 32 us with the averaged cells and the ghost cells found by ballots and
+// dealt to the lanes (bound by scattered lines: both sets use a part of each).
 // ---------------------------------------------------------------------------------------------
 template <typename T, typename S, int Q, bool FOLD>
 __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const int *__restrict__ ids, int n, S *Fp, S *Fc,
@@ -299,8 +405,19 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const in
         fc = nbr_child[b];
         work = fc >= 0 && blk_mask[b] == BLK_INTERFACE;
     }
-    // ---- average: NCH lanes per parent cell, two parent cells per lane group (k_average) ----
-    {
+    // ---- average (k_average) ----
+    if constexpr (DIM == 3) {
+        if (work) {  // the same for the whole workgroup
+            const unsigned long long done = average_block_3d<T, S, Q>(
+                Fc, ncm, cells_mask, fc, 0, ratio_avg, s_red, [&](int ta, int p, T v) {
+                    const T wq = (T)VelSet<Q>::w(p);
+                    const S enc = ST::enc(v, wq);
+                    Fp[(long long)p * ncm + (long long)b * CELLS + ta] = enc;
+                    s_avg[p * CELLS + ta] = ST::dec(enc, wq);
+                });
+            if (threadIdx.x < CELLS) s_done[threadIdx.x] = (int)((done >> threadIdx.x) & 1);
+        }
+    } else {
         const int k = r % NCH, ta0 = r / NCH;  // parent cells ta0 and ta0 + CELLS / 2
         const int off = (k & 1) + 4 * ((k >> 1) & 1) + 16 * ((k >> 2) & 1);
         bool avg[2];
@@ -359,9 +476,12 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const in
         }
     }
     // The children's cell masks for the interpolation stage, fetched before the barrier.
+    __shared__ GhostList s_ghost;
     const int c = r / CELLS, t = r % CELLS;
     bool put[2] = {false, false};
-    if (work)
+    if constexpr (DIM == 3)
+        ghost_masks(s_ghost, cells_mask, fc, work);
+    else if (work)
 #pragma unroll
         for (int h = 0; h < 2; h++) put[h] = cells_mask[(long long)(fc + c + h * HALF) * CELLS + t] == CELL_GHOST;
     __syncthreads();
@@ -384,10 +504,19 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const in
             sg[p * PPW * CELLS + t] = fe + (f[p] - fe) * ratio_int;
         }
     }
+    int total = 0;
+    if constexpr (DIM == 3) total = ghost_list(s_ghost);
     __syncthreads();
     interp_coefficients<T, Q, PPW, IWG>(s_all, s_coef);
     __syncthreads();
     if (!work) return;
+    if constexpr (DIM == 3) {
+        for (int e = threadIdx.x; e < total; e += IWG) {
+            const int x = s_ghost.cell[e];
+            interp_child<T, S, Q>(s_coef, x >> 6, x & 63, Fc, ncm, (long long)fc * CELLS + x);
+        }
+        return;
+    }
 #pragma unroll
     for (int h = 0; h < 2; h++)
         if (put[h])
@@ -601,12 +730,14 @@ __global__ __launch_bounds__(CWG) void k_interp_cubic(InterpArgs<T, S> ia)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Fine -> coarse: Cu_Average (solver_lbm_kernels_comm.cu:174-347).  NG consecutive lanes (NG = 8
-// in 3D, 4 in 2D) serve one parent cell, each lane loading and rescaling one child cell of the
-// cell's 2x2(x2) group; the group sum is formed in the reference's order from the NG lanes by
-// shuffles and each lane stores the directions p = lane (mod NG).  Each lane group serves two
-// parent cells (t and t + CELLS/2, both loaded before either is reduced), which halves the
-// wavefronts per parent.  No LDS, no barriers.
+// Fine -> coarse: Cu_Average (solver_lbm_kernels_comm.cu:174-347).  3D: one workgroup per parent block
+// (average_block_3d), bound by the children's interface cells, 1/8 of every row's lines used; finding the
+// averaged cells by a ballot instead of serving all 64: 17.6 -> 14.2 us for 3008 parents, 8.3 -> 6.0 us
+// for 736, 300 -> 284 us for 48 896 (D3Q19 FP32).  2D: NG = 4 consecutive lanes serve one parent cell, each
+// lane loading and rescaling one child cell of the cell's 2x2 group; the group sum is formed in the
+// reference's order from the NG lanes by shuffles and each lane stores the directions p = lane (mod NG).
+// Each lane group serves two parent cells (t and t + CELLS/2, both loaded before either is reduced), which
+// halves the wavefronts per parent.
 // ---------------------------------------------------------------------------------------------
 template <typename T, typename S, int Q, bool FOLD>
 __global__ __launch_bounds__(WG) void k_average(FixupArgs<T, S> fa, const int *__restrict__ ids, int n, S *Fp,
@@ -620,6 +751,15 @@ __global__ __launch_bounds__(WG) void k_average(FixupArgs<T, S> fa, const int *_
     constexpr int NG = (DIM == 3) ? 8 : 4;     // child cells per parent cell
     constexpr int PER_BLOCK = CELLS / 2 * NG;   // lanes per parent block: two parent cells per lane group
     __shared__ T s_red[(WG / 64) * Q * 65];     // per-wavefront rows of the group sums
+    if constexpr (DIM == 3) {
+        const int pb = ids[blockIdx.x], pfc = nbr_child[pb];
+        // The same for the whole workgroup.
+        if (pfc < 0 || !(ave_type == 2 || blk_mask[pb] == BLK_INTERFACE)) return;
+        average_block_3d<T, S, Q>(Fc, ncm, cells_mask, pfc, ave_type, tau_ratio, s_red, [&](int t, int p, T v) {
+            Fp[(long long)p * ncm + (long long)pb * CELLS + t] = Store<T, S>::enc(v, (T)VelSet<Q>::w(p));
+        });
+        return;
+    }
     const int k = threadIdx.x % NG;             // which child cell of the group
     const long long gid = (long long)blockIdx.x * WG + threadIdx.x;
     const long long bi = gid / PER_BLOCK;
@@ -717,7 +857,8 @@ __global__ __launch_bounds__(WG, (COLL == COLL_MRT && Q == 27 && sizeof(T) == 4 
     // rows and coefficients, or the matrix-core MRT's per-wavefront transpose rows.
     constexpr int ROW = Store<T, S>::quantized ? 20 : 36;
     constexpr int ALL16 = (IL::ALL * (int)sizeof(T) + 15) / 16 * 16 / (int)sizeof(T);  // coefficients 16-byte aligned
-    constexpr size_t INTERP_BYTES = sizeof(T) * (ALL16 + IL::COEF);
+    constexpr size_t GHOSTS = (sizeof(T) * (ALL16 + IL::COEF) + 15) / 16 * 16;
+    constexpr size_t INTERP_BYTES = GHOSTS + (VS::DIM == 3 ? sizeof(GhostList) : 0);
     constexpr size_t MRT_BYTES = MF ? sizeof(float) * (WG / 64) * 64 * ROW : 0;
     __shared__ __attribute__((aligned(16))) unsigned char s_raw[INTERP_BYTES > MRT_BYTES ? INTERP_BYTES : MRT_BYTES];
     if constexpr (FOLD) resolve_pending<T, S, Q>(x.fa);
@@ -725,7 +866,7 @@ __global__ __launch_bounds__(WG, (COLL == COLL_MRT && Q == 27 && sizeof(T) == 4 
         if ((int)blockIdx.x < x.interp_wgs) {
             T *s_all = reinterpret_cast<T *>(s_raw);
             T *s_coef = s_all + ALL16;
-            interp_parents<T, S, Q, false>(x.ia, blockIdx.x, s_all, s_coef);
+            interp_parents<T, S, Q, false>(x.ia, blockIdx.x, s_all, s_coef, *reinterpret_cast<GhostList *>(s_raw + GHOSTS));
         }
         return;
     }
