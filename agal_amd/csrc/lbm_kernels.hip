@@ -871,15 +871,14 @@ __global__ __launch_bounds__(WG, (COLL == COLL_MRT && Q == 27 && sizeof(T) == 4 
         return;
     }
     const int wg = (int)blockIdx.x - x.lead;
-    const int slot = __builtin_amdgcn_readfirstlane(xcd_local_wg(wg, x.step_wgs) * (WG / 64) + (int)(threadIdx.x >> 6));
-    if (slot >= m.start[m.nlv]) return;  // whole wavefronts only; the fused step has no barrier
     int k = 0;
 #pragma unroll
     for (int j = 1; j < MAXLV; j++)
-        if (j < m.nlv && slot >= m.start[j]) k = j;
+        if (j < m.nlv && wg >= m.start[j]) k = j;
     k = __builtin_amdgcn_readfirstlane(k);
     const StepArgs<T, S> &a = m.lv[k];
-    const int wave = slot - m.start[k];
+    const int wave = __builtin_amdgcn_readfirstlane(xcd_local_wg(wg - m.start[k], m.start[k + 1] - m.start[k]) * (WG / 64) +
+                                                    (int)(threadIdx.x >> 6));
     if constexpr (VS::DIM == 3) {
         // One transpose region per wavefront for the matrix-core MRT: 64 rows of 36 floats, or of
         // 20 floats (80 bytes: the forward rows, and the back rows in binary16) with 16-bit pools.
@@ -1437,7 +1436,7 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
         MultiStep<T, S> m;
         StepExtras<T, S> x;
         m.nlv = 0;
-        long long waves = 0;
+        int wgs = 0;
         double cells = 0;
         unsigned rmask = 0, wmask = 0;
         bool finest = false;
@@ -1452,13 +1451,14 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
             if (first < 0) first = L;
             m.lv[m.nlv] = step_args<T, S, Q>(c, L, rd[j], mode);
             m.lv[m.nlv].skip_linked = link_step_due(c, L);
-            m.start[m.nlv] = (int)waves;
-            waves += (n + BPW - 1) / BPW;
+            m.start[m.nlv] = wgs;
+            const int waves = (n + BPW - 1) / BPW;
+            wgs += ((waves + WG / 64 - 1) / (WG / 64) + 7) / 8 * 8;  // a multiple of the XCD count
             cells += (double)n * CELLS;
             m.nlv++;
         }
-        for (int k = m.nlv; k <= MAXLV; k++) m.start[k] = (int)waves;
-        x.step_wgs = m.nlv ? (int)((waves + WG / 64 - 1) / (WG / 64) + 7) / 8 * 8 : 0;  // a multiple of the XCD count
+        for (int k = m.nlv; k <= MAXLV; k++) m.start[k] = wgs;
+        x.step_wgs = wgs;
         x.interp_wgs = 0;
         if (base == 0) {
             if (ia && ia->n > 0) {
