@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -192,7 +193,7 @@ struct Ctx {
         pending_fix.push_back({L, buf, exchange, exc_slot(L)});
         exc_turn[L] ^= 1;
     }
-    // 1 while the first, 2 while the second sub-step of a finest-level pair is issued, else 0.
+    // 1 while the first, 2 while the second sub-step of a pair is issued, else 0.
     int fine_pair = 0;
     hipStream_t lstream[8] = {};
     bool slot_joined[NSLOT] = {};
@@ -205,6 +206,12 @@ struct Ctx {
     int *id_set_L(int L) const { return id_set + (size_t)L * n_maxcblocks; }
     int *order_L(int L) const { return order + (size_t)L * n_maxcblocks; }
     int *iface_L(int L) const { return iface + (size_t)L * n_maxcblocks; }
+
+    // Pinned pieces of large downloads (download_rows, capi.hip), made by the first one.
+    static constexpr int DL_SLOTS = 8;
+    void *dl_stage = nullptr;
+    hipEvent_t dl_ev[DL_SLOTS] = {};
+    std::mutex dl_mu;
 };
 
 // Records the HIP error text and returns AGAL_ERR_HIP.

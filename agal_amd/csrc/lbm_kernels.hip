@@ -16,8 +16,8 @@
 //   - a link (x -> x+c_h, h in the reference's half set) streams when x collides and the
 //     partner's f*_{pb(h)} > 0; otherwise both ends bounce back into their own opposite slot.
 //     The partner knows its value, the initiator does not: the initiator always pushes, and a
-//     partner whose value fails the guard records the link in an exception list that a one-
-//     workgroup fix-up kernel resolves after the step (normally empty).
+//     partner whose value fails the guard records the link in an exception list (normally empty) that
+//     is resolved before anything else reads the level: by the next kernel, or by k_fixup.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -48,7 +48,6 @@ __global__ __launch_bounds__(WG) void k_set_ic(const int *__restrict__ ids, int 
         F[(long long)p * ncm + cell] = Store<T, S>::enc(f, (T)VS::w(p));
     }
 }
-
 
 template <typename T, typename S, int Q>
 __global__ __launch_bounds__(WG) void k_refresh(const int *__restrict__ ids, int n, const S *__restrict__ F,

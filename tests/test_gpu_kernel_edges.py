@@ -3,9 +3,11 @@ of their ranges, against the CPU restatement."""
 from __future__ import annotations
 
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
+import torch
 
 from agal_amd import capi
 from agal_amd.mesh import LbmMesh
@@ -126,3 +128,31 @@ def test_pending_lists_resolved_by_the_next_kernel(vs, prec):
         bad = compare_states(g.state(), o.state())
         assert not bad, "\n".join(bad)
     g.close()
+
+
+@pytest.mark.parametrize("vs,prec,N,nb", [(capi.D3Q19, capi.FP32, 60, 4095), (capi.D3Q19, capi.FP32, 60, 4096),
+                                          (capi.D3Q27, capi.FP64, 76, 8200), (capi.D2Q9, capi.FP16, 508, 16385)])
+def test_large_downloads_in_pieces(vs, prec, N, nb):
+    """Macroscopic fields and populations around the line between a direct copy and pinned pieces (4 MB),
+    and rows that end within a piece: into pageable memory with a gap between the rows, into pinned memory
+    (copied directly), and from two threads at once.  All must hold the same bytes; the gaps stay as they
+    were."""
+    m = LbmMesh(ldc_params(vs=vs, N=N, Re=40.0, levels=1, prec=prec), nb)
+    q, nc = m.sizes.n_q, nb * m.sizes.cells_per_block
+    m.set_populations(np.random.default_rng(nb).uniform(0.5 / q, 1.5 / q, (q, nc)))
+    m.S_RefreshVariables(0)
+    for what, rows in (("download_macros", 4), ("download_populations", q)):
+        pinned = torch.full((rows, nc), -7.0, dtype=torch.float64 if m.dtype == np.float64 else torch.float32, pin_memory=True)
+        m._call(what, capi.np_ptr(pinned.numpy()), nb, nc)
+        ref = pinned.numpy().view(np.uint8)
+        assert ref.any()
+
+        def check():
+            out = np.full((rows, nc + 3), -7, dtype=m.dtype)
+            m._call(what, capi.np_ptr(out), nb, nc + 3)
+            return np.array_equal(out[:, :nc].copy().view(np.uint8), ref) and bool((out[:, nc:] == -7).all())
+
+        assert check()
+        with ThreadPoolExecutor(2) as pool:
+            assert all(f.result() for f in [pool.submit(check) for _ in range(4)])
+    m.close()
