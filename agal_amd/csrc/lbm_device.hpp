@@ -1021,8 +1021,8 @@ __device__ __forceinline__ void fixup_reset(const FixupArgs<T, S> &fa, int lv)
 // any list holds an entry, the workgroup that draws ticket 0 resolves all lists and raises the flag, the
 // others wait for it -- a workgroup that runs, so the wait ends whatever the order of dispatch -- and the
 // last one to pass empties the lists and the counters of this hand-over.  The kernel records into other
-// lists than it resolves here, so every workgroup finds the counters as the first did.  Called by all
-// threads of all workgroups, before any exit, in the FOLD variants of the kernels (its mere presence
+// lists than it resolves here (fold_fixups sees to it), so every workgroup finds the counters as the first
+// did.  Called by all threads of all workgroups, before any exit, in the FOLD variants of the kernels (its mere presence
 // costs a large launch 1-3%).  With entries the hand-over takes 10-15 us, and the
 // acquire of a workgroup that starts later empties the L2 under those that run (64^3 cavity, launches
 // of 6016 workgroups, 130 entries: 547 us a coarse step against 292), so only launches that are bound by
@@ -1192,13 +1192,30 @@ static inline int launch_fixups_for(Ctx *c, unsigned touch)
     return AGAL_OK;
 }
 
-// The pending lists for a launch of `wgs` workgroups that touches the levels in `touch`: all handed to it
-// in fa, or, for a large launch that touches one of them, all resolved by a fixup launch before it.
+// Lists (bits, numbered as in exc_count) that the sub-step of level L in mode `vmode` records into.
+static inline unsigned long long records_into(const Ctx *c, int L, int vmode)
+{
+    return 1ull << (vmode == 1 ? c->exc_extra() : c->exc_slot(L));
+}
+
+// The pending lists for a launch of `wgs` workgroups that touches the levels in `touch` and records into
+// the lists in `records`: all handed to it in fa, or, for a large launch that touches one of them, all
+// resolved by a fixup launch before it.  A launch never resolves a list that it records into: its
+// workgroups would find different counters.  A level's own two lists take turns, but the extra list,
+// emptied with the pending list of the finest level's second sub-step, is recorded into by the next first
+// one, and nothing lies between the two where the parent level is refined as a whole (no interface
+// blocks, hence no average).
 template <typename T, typename S, int Q>
-static inline int fold_fixups(Ctx *c, int wgs, unsigned touch, FixupArgs<T, S> &fa, unsigned &wmask)
+static inline int fold_fixups(Ctx *c, int wgs, unsigned touch, unsigned long long records, FixupArgs<T, S> &fa, unsigned &wmask)
 {
     const bool fold = wgs <= FOLD_MAX_WGS;
-    if (!fold || c->pending_fix.size() > MAXLV)
+    unsigned long long resolves = 0;
+    for (const auto &pf : c->pending_fix) {
+        resolves |= 1ull << pf.slot;
+        if (pf.L == c->MAX_LEVELS - 1) resolves |= 1ull << c->exc_extra();
+    }
+    if (resolves & records) touch = ~0u;
+    if (!fold || c->pending_fix.size() > MAXLV || (resolves & records))
         if (int st = launch_fixups_for<T, S, Q>(c, touch)) return st;
     take_fixups<T, S>(c, fold ? ~0u : 0u, fa, wmask);
     return AGAL_OK;

@@ -111,7 +111,7 @@ static int odd_step_t(Ctx *c, int L)
         FixupArgs<T, S> fa;
         unsigned rmask = res_bit(L, buf), wmask = rmask;
         const int grid = ((n + WG / 64 - 1) / (WG / 64) + 7) / 8 * 8;  // a multiple of the XCD count
-        if (int st = fold_fixups<T, S, Q>(c, grid, 1u << L, fa, wmask)) return st;
+        if (int st = fold_fixups<T, S, Q>(c, grid, 1u << L, records_into(c, L, 0), fa, wmask)) return st;
         hipStream_t s = sched_begin(c, 0, rmask, wmask);
         const bool mrt = c->P.collision == AGAL_MRT;
         using K = void (*)(StepArgs<T, S>, FixupArgs<T, S>);

@@ -1438,6 +1438,7 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
         int wgs = 0;
         double cells = 0;
         unsigned rmask = 0, wmask = 0;
+        unsigned long long records = 0;
         bool finest = false;
         int first = -1;
         for (int j = base; j < nl && j < base + MAXLV; j++) {
@@ -1449,6 +1450,7 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
             finest = finest || L == c->MAX_LEVELS - 1;
             if (first < 0) first = L;
             m.lv[m.nlv] = step_args<T, S, Q>(c, L, rd[j], mode);
+            records |= records_into(c, L, mode);
             m.lv[m.nlv].skip_linked = link_step_due(c, L);
             m.start[m.nlv] = wgs;
             const int waves = (n + BPW - 1) / BPW;
@@ -1470,7 +1472,7 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
         x.lead = (x.interp_wgs + 7) / 8 * 8;
         if (x.step_wgs + x.interp_wgs == 0) continue;
         const int grid = x.lead + x.step_wgs;
-        if ((st = fold_fixups<T, S, Q>(c, grid, touch, x.fa, wmask))) return st;
+        if ((st = fold_fixups<T, S, Q>(c, grid, touch, records, x.fa, wmask))) return st;
         const int slot = (finest || m.nlv != 1 || x.interp_wgs || x.fa.n) ? 0 : 1 + first;
         hipStream_t s = sched_begin(c, slot, rmask, wmask);
         // One kernel per collision operator: BGK alone needs fewer registers than MRT's moments.  The
@@ -1621,7 +1623,7 @@ static int average_t(Ctx *c, int L, int var)
     unsigned wl = res_bit(L, c->cur[L]);
     FixupArgs<T, S> fa;
     const int grid = nwg(n, VelSet<Q>::CELLS / 2 * (VelSet<Q>::DIM == 3 ? 8 : 4));
-    if (int st = fold_fixups<T, S, Q>(c, grid, 3u << L, fa, wl)) return st;
+    if (int st = fold_fixups<T, S, Q>(c, grid, 3u << L, 0, fa, wl)) return st;
     hipStream_t s = sched_begin(c, 0, rl, wl);
     hipLaunchKernelGGL((fa.n ? k_average<T, S, Q, true> : k_average<T, S, Q, false>), dim3(grid), dim3(WG), 0, s, fa, ids, n, Fbuf<S>(c, c->cur[L]), Fbuf<S>(c, c->cur[L + 1]), c->n_maxcells, c->nbr_child,
                        c->blk_mask, c->cells_mask, var, ratio);
@@ -1643,7 +1645,7 @@ static int avg_interp_t(Ctx *c, int L)
     const T ratio_int = (T)c->tau_vec[L + 1] / (T)c->tau_vec[L];
     unsigned m = res_bit(L, c->cur[L]) | res_bit(L + 1, c->cur[L + 1]);
     FixupArgs<T, S> fa;
-    if (int st = fold_fixups<T, S, Q>(c, interp_grid<Q>(n), 3u << L, fa, m)) return st;
+    if (int st = fold_fixups<T, S, Q>(c, interp_grid<Q>(n), 3u << L, 0, fa, m)) return st;
     hipStream_t s = sched_begin(c, 0, m, m);
     hipLaunchKernelGGL((fa.n ? k_avg_interp<T, S, Q, true> : k_avg_interp<T, S, Q, false>), dim3(interp_grid<Q>(n)), dim3(IWG), 0, s, fa, c->iface_L(L), n,
                        Fbuf<S>(c, c->cur[L]), Fbuf<S>(c, c->cur[L + 1]), c->n_maxcells, c->nbr_child, c->blk_mask,
