@@ -480,11 +480,12 @@ __global__ __launch_bounds__(AWG) void k_update_masks_2(int *cells_mask, const i
 // Slot-ordered neighbour table, participation flag and solid-cell flag per block: a workgroup takes
 // 64 blocks, reads their tables by rows and writes them as one run through LDS, and their cell masks as
 // one run (a thread per block, each walking its own 256 bytes: 90 us for 0.55 M blocks, 24 so).
-// traits: participation (bit 0), solid cells (bit 1), level << 2.
+// traits: participation (bit 0), solid cells (bit 1), level << 2, where a level outside 0 .. ml - 1 (the tables can
+// be uploaded, and children of the finest level can be asked for) counts as ml: in no level's list.
 template <int DIM>
 __global__ __launch_bounds__(AWG) void k_block_aux(const int *nbr, const int *nbr_child, const int *blk_mask,
                                                    const int *cells_mask, const int *level, int *nbr_slot, int *part,
-                                                   int *traits, long long nmax, int n)
+                                                   int *traits, long long nmax, int n, int ml)
 {
     constexpr int CELLS = DIM == 3 ? 64 : 16, QMAX = DIM == 3 ? 27 : 9, NB = 64;
     __shared__ int s_nbr[NB * QMAX], s_solid[NB];
@@ -505,8 +506,9 @@ __global__ __launch_bounds__(AWG) void k_block_aux(const int *nbr, const int *nb
     if ((int)threadIdx.x < nb) {
         const int kap = k0 + threadIdx.x;
         const int pt = (nbr_child[kap] < 0 || blk_mask[kap] != BLK_SOLID) ? 1 : 0;
+        const int lv = level[kap];
         part[kap] = pt;
-        traits[kap] = pt | (s_solid[threadIdx.x] << 1) | (level[kap] << 2);
+        traits[kap] = pt | (s_solid[threadIdx.x] << 1) | ((lv >= 0 && lv < ml ? lv : ml) << 2);
     }
 }
 
@@ -519,7 +521,7 @@ __global__ __launch_bounds__(AWG) void k_block_aux(const int *nbr, const int *nb
 // Half a wavefront (2D: a quarter) per block, a lane per slot.
 template <int DIM>
 __global__ __launch_bounds__(AWG) void k_block_simple(const int *nbr_slot, const int *traits, const int *ref, int *simple,
-                                                      int n, int max_nz, int *n_general)
+                                                      int n, int max_nz, int *n_general, int ml)
 {
     constexpr int QMAX = DIM == 3 ? 27 : 9, LN = DIM == 3 ? 32 : 16;
     const int lane = threadIdx.x & 63, S = lane % LN, g0 = lane - S;
@@ -541,7 +543,7 @@ __global__ __launch_bounds__(AWG) void k_block_simple(const int *nbr_slot, const
     if (!act || S != 0) return;
     const int s = (mine & 3) != 1 || any_bad ? 0 : (!any_gone && is_self ? 2 : 1);
     simple[kap] = s;
-    if ((s == 0 || any_strange) && ref[kap] != REF_INACTIVE) atomicAdd(&n_general[mine >> 2], 1);
+    if ((s == 0 || any_strange) && (mine >> 2) < ml && ref[kap] != REF_INACTIVE) atomicAdd(&n_general[mine >> 2], 1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -842,14 +844,14 @@ int rebuild_level_lists(Ctx *c, long long range_hint)
     const dim3 aux((n + 63) / 64), blk(AWG);
     if (c->DIM == 3) {
         hipLaunchKernelGGL((k_block_aux<3>), aux, blk, 0, c->stream, c->nbr, c->nbr_child, c->blk_mask, c->cells_mask,
-                           c->level, c->nbr_slot, c->part, c->scan_a, c->n_maxcblocks, n);
+                           c->level, c->nbr_slot, c->part, c->scan_a, c->n_maxcblocks, n, ML);
         hipLaunchKernelGGL((k_block_simple<3>), dim3(grid1(32LL * n)), blk, 0, c->stream, c->nbr_slot, c->scan_a, c->ref,
-                           c->simple, n, c->Q == 27 ? 3 : 2, c->dscal + 24);
+                           c->simple, n, c->Q == 27 ? 3 : 2, c->dscal + 24, ML);
     } else {
         hipLaunchKernelGGL((k_block_aux<2>), aux, blk, 0, c->stream, c->nbr, c->nbr_child, c->blk_mask, c->cells_mask,
-                           c->level, c->nbr_slot, c->part, c->scan_a, c->n_maxcblocks, n);
+                           c->level, c->nbr_slot, c->part, c->scan_a, c->n_maxcblocks, n, ML);
         hipLaunchKernelGGL((k_block_simple<2>), dim3(grid1(16LL * n)), blk, 0, c->stream, c->nbr_slot, c->scan_a, c->ref,
-                           c->simple, n, 2, c->dscal + 24);
+                           c->simple, n, 2, c->dscal + 24, ML);
     }
     AGAL_HIP(c, hipGetLastError());
     if ((st = build_traversal_order(c))) return st;

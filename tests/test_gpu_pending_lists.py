@@ -69,3 +69,38 @@ def test_finest_pairs_under_a_wholly_refined_level(vs, prec, coll, amp, graphs):
     _perturb(g, o, amp)
     _step_and_compare(g, o, (1, 2, 1))
     g.close()
+
+
+@pytest.mark.parametrize("lv", [2, 7, 8, 9, 40, 1 << 29, (1 << 31) - 1, -1, -(1 << 31)])
+def test_a_block_of_no_level_is_in_no_list(lv):
+    """An uploaded block table may hold any level.  A block whose level is none of the mesh's is left out of
+    every list: the averages and interpolations of the others are the restatement's, and with its level
+    back the mesh steps as if nothing had been."""
+    p = ldc_params(vs=capi.D3Q19, N=16, Re=40.0, levels=2, P_REFINE=1 << 28)
+    g, o, q = LbmMesh(p, 1024), OracleMesh(p, 1024), OracleMesh(p, 1024)
+    for m in (g, o):
+        m.S_SetIC(0)
+        ids = m.id_set(0)
+        m.mark_blocks(ids[m.coords()[0, ids] < 0.3], capi.REF_MARK_REFINE)
+        m.M_RefineAndCoarsenBlocks()
+        m.advance_loop(0, 3)
+    st = o.state()
+    fine = st["id_sets"][1]
+    level, b = st["level"].copy(), int(fine[len(fine) // 2])
+    level[b] = lv
+    g.set_block_ints(capi.BLK_LEVEL, level)
+    sets = [st["id_sets"][0], fine[fine != b]]
+    assert [g.id_set(L).tolist() for L in range(2)] == [s.tolist() for s in sets]
+    q.import_state(dict(st, level=level, id_sets=sets, n_ids=[len(s) for s in sets]))
+    for m in (g, q):
+        m.S_Interpolate(0, capi.INTERP_INTERFACE)
+        m.S_Average(0, capi.AVERAGE_INTERFACE)
+    cells = (64 * np.concatenate(sets)[:, None] + np.arange(64)).ravel()
+    np.testing.assert_array_equal(g.populations(st["id_max"])[:, cells], q.populations(st["id_max"])[:, cells])
+    g.set_block_ints(capi.BLK_LEVEL, st["level"])
+    g.set_populations(st["f"])
+    for m in (g, o):
+        m.advance_loop(3, 3)
+    bad = compare_states(g.state(), o.state())
+    assert not bad, "\n".join(bad)
+    g.close()
