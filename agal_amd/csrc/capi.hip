@@ -381,14 +381,15 @@ int advance_step(Ctx *c, int L0)
     return launch_mea_post(c);
 }
 
-// `k` consecutive coarse steps from level L0.  Without refinement the steps have nothing between them:
-// each resolves the exception list of the one before as it starts, and two at a time run as in-place
-// pairs where the level allows it.
+// `k` consecutive coarse steps from level L0.  Without refinement (a step from the finest level of a
+// refined mesh is two sub-steps, advance_rec's) the steps have nothing between them: each resolves the
+// exception list of the one before as it starts, and two at a time run as in-place pairs where the level
+// allows it.
 int advance_steps(Ctx *c, int L0, int k)
 {
     int st = AGAL_OK;
-    const bool multi = c->MAX_LEVELS > 1 && c->MAX_LEVELS != L0 + 1;
-    if (!multi && !c->cv_F && !c->links_on) {
+    const bool one_level = L0 == c->MAX_LEVELS - 1 && (c->MAX_LEVELS == 1 || L0 == c->N_LEVEL_START);
+    if (one_level && !c->cv_F && !c->links_on) {
         const bool pairs = inplace_pair(c, L0);
         c->defer_coarse = true;
         while (k > 0 && st == AGAL_OK) {
