@@ -12,6 +12,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <optional>
 #include <string>
 #include <thread>
 #include <vector>
@@ -1486,10 +1487,30 @@ static bool dl_prepare(Ctx *c, const void *dst)
     return true;
 }
 
+// Makes the context's GPU current for a scope.  A direct copy needs only its stream; the pieces and their
+// events have to be made on the stream's GPU, whichever one the calling thread has current.
+struct DeviceScope {
+    int prev = -1, device;
+    bool ok;
+    explicit DeviceScope(int dev) : device(dev)
+    {
+        ok = hipGetDevice(&prev) == hipSuccess && (prev == device || hipSetDevice(device) == hipSuccess);
+        if (!ok) (void)hipGetLastError();
+    }
+    ~DeviceScope()
+    {
+        if (prev >= 0 && prev != device) (void)hipSetDevice(prev);
+    }
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+};
+
 static int download_rows(Ctx *c, void *dst, size_t dst_pitch, const void *src, size_t src_pitch, size_t bytes, int rows)
 {
     std::unique_lock<std::mutex> pieces_free(c->dl_mu, std::defer_lock);  // another thread's download has them: as it was
-    if (bytes * rows < DL_MIN || !pieces_free.try_lock() || !dl_prepare(c, dst)) {
+    std::optional<DeviceScope> gpu;
+    if (bytes * rows >= DL_MIN) gpu.emplace(c->device);
+    if (!gpu || !gpu->ok || !pieces_free.try_lock() || !dl_prepare(c, dst)) {
         for (int r = 0; r < rows; r++)
             AGAL_HIP(c, hipMemcpyAsync((char *)dst + r * dst_pitch, (const char *)src + r * src_pitch, bytes,
                                        hipMemcpyDeviceToHost, c->stream));
