@@ -1357,9 +1357,22 @@ static bool mea_due(const Ctx *c, int L)
     return !multi || c->global_Liter == (1 << (c->MAX_LEVELS - 1)) - 1;
 }
 
+// The collision operator of the fused step's launches.
+template <typename T, int Q>
+static int fused_operator(const Ctx *c)
+{
+    if (c->P.collision != AGAL_MRT) return COLL_BGK;
+    return sizeof(T) == 4 && VelSet<Q>::DIM == 3 && c->mrt_mfma ? COLL_MFMA : COLL_MRT;
+}
+
+// Whether the linked blocks' sub-step is k_link_step's: where its rules differ from the fused step's, and
+// where its collision does -- on matrix cores the fused step's MRT is of another precision, and a block
+// near the wall would alternate between the two from one sub-step to the next.
+template <typename T, int Q>
 static bool link_step_due(const Ctx *c, int L)
 {
-    return c->links_on && c->lk_n[L] > 0 && (c->P.S_BC_TYPE == 1 || mea_due(c, L));
+    return c->links_on && c->lk_n[L] > 0 &&
+           (c->P.S_BC_TYPE == 1 || mea_due(c, L) || fused_operator<T, Q>(c) == COLL_MFMA);
 }
 
 template <typename T>
@@ -1382,13 +1395,13 @@ static LinkArgs<T> link_args(Ctx *c, int L, bool mea)
 }
 
 // The linked blocks' sub-step of level L reading buffer rd, on stream s, where it differs from that of
-// other blocks: with the interpolated bounce-back, or when the momentum exchange is due.  Otherwise the
-// fused step takes the linked blocks like any (link_step_due).
+// other blocks: with the interpolated bounce-back, when the momentum exchange is due, or with the fused
+// step's MRT on matrix cores.  Otherwise the fused step takes the linked blocks like any (link_step_due).
 template <typename T, typename S, int Q>
 static int launch_link_step(Ctx *c, int L, int rd, hipStream_t s)
 {
     if constexpr (VelSet<Q>::DIM == 3) {
-        if (!link_step_due(c, L)) return AGAL_OK;
+        if (!link_step_due<T, Q>(c, L)) return AGAL_OK;
         const LinkArgs<T> la = link_args<T>(c, L, mea_due(c, L));
         const bool fm = la.bc_type == 1 || (la.mea && la.order != 1);
         hipLaunchKernelGGL((fm ? k_link_step<T, S, Q, true> : k_link_step<T, S, Q, false>),
@@ -1451,7 +1464,7 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
             if (first < 0) first = L;
             m.lv[m.nlv] = step_args<T, S, Q>(c, L, rd[j], mode);
             records |= records_into(c, L, mode);
-            m.lv[m.nlv].skip_linked = link_step_due(c, L);
+            m.lv[m.nlv].skip_linked = link_step_due<T, Q>(c, L);
             m.start[m.nlv] = wgs;
             const int waves = (n + BPW - 1) / BPW;
             wgs += ((waves + WG / 64 - 1) / (WG / 64) + 7) / 8 * 8;  // a multiple of the XCD count
@@ -1478,11 +1491,12 @@ static int launch_fused(Ctx *c, const int *levels, const int *rd, int nl, const 
         // One kernel per collision operator: BGK alone needs fewer registers than MRT's moments.  The
         // matrix-core MRT variant: FP32 compute, 3D sets, when enabled.
         using K = void (*)(MultiStep<T, S>, StepExtras<T, S>);
-        const bool mrt = c->P.collision == AGAL_MRT, fold = x.fa.n > 0;
+        const int op = fused_operator<T, Q>(c);
+        const bool mrt = op != COLL_BGK, fold = x.fa.n > 0;
         K kern = mrt ? (fold ? (K)k_collide_stream<T, S, Q, COLL_MRT, true> : (K)k_collide_stream<T, S, Q, COLL_MRT, false>)
                      : (fold ? (K)k_collide_stream<T, S, Q, COLL_BGK, true> : (K)k_collide_stream<T, S, Q, COLL_BGK, false>);
         if constexpr (sizeof(T) == 4 && VelSet<Q>::DIM == 3)
-            if (mrt && c->mrt_mfma)
+            if (op == COLL_MFMA)
                 kern = fold ? (K)k_collide_stream<T, S, Q, COLL_MFMA, true> : (K)k_collide_stream<T, S, Q, COLL_MFMA, false>;
         if ((st = launch_timed(c, kern, grid, s, cells, m, x))) return st;
         for (int j = base; j < nl && j < base + MAXLV; j++)
