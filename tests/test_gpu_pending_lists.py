@@ -22,7 +22,7 @@ def _refined_pair(vs, prec, coll, N, x_max, solid):
     `solid`, two cells of the finest level turned solid, which keeps its sub-steps out of the in-place form."""
     p = ldc_params(vs=vs, N=N, Re=40.0, levels=3, P_REFINE=1 << 28, prec=prec, collision=coll)
     p.L_fy = p.L_fz = 0.5
-    g, o = LbmMesh(p, 4096), OracleMesh(p, 4096)
+    g, o = LbmMesh(p, 16384), OracleMesh(p, 16384)  # lists of 2^20 entries
     for m in (g, o):
         m.S_SetIC(0)
         for L in range(2):
@@ -103,4 +103,19 @@ def test_a_block_of_no_level_is_in_no_list(lv):
         m.advance_loop(3, 3)
     bad = compare_states(g.state(), o.state())
     assert not bad, "\n".join(bad)
+    g.close()
+
+
+@pytest.mark.parametrize("vs,prec,coll,amp", SETS)
+@pytest.mark.parametrize("N,x_max,solid", [(16, 0.3, True), (16, 0.3, False), (16, 9.0, True)])
+def test_finest_pairs_with_failed_links(vs, prec, coll, amp, N, x_max, solid):
+    """Many failed links on every level.  With solid cells on the finest level its pairs are push pairs: the
+    first sub-step links its entries per block and flags the blocks, the second applies them as it loads; 256
+    blocks in launches that resolve what is pending themselves, and 1024 blocks, whose launches leave that to
+    a fixup launch.  Without solid cells 256 blocks step in place, and the second sub-step resolves the first
+    one's list."""
+    g, o = _refined_pair(vs, prec, coll, N, x_max, solid)
+    assert int(g.sizes.n_ids[2]) == (256 if x_max < 1 else 1024)
+    _perturb(g, o, amp)
+    _step_and_compare(g, o, (1, 2, 1))
     g.close()
