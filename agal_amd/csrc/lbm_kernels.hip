@@ -418,17 +418,16 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const in
         }
     } else {
         const int k = r % NCH, ta0 = r / NCH;  // parent cells ta0 and ta0 + CELLS / 2
-        const int off = (k & 1) + 4 * ((k >> 1) & 1) + 16 * ((k >> 2) & 1);
+        const int off = (k & 1) + 4 * (k >> 1);
         bool avg[2];
         long long cb[2];
         int c0[2];
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int ta = ta0 + h * (CELLS / 2);
-            const int I = ta % 4, J = (ta / 4) % 4, K = (DIM == 3) ? ta / 16 : 0;
-            const int cq = (I / 2) + 2 * (J / 2) + 4 * (K / 2);
+            const int I = ta % 4, J = ta / 4;
+            const int cq = (I / 2) + 2 * (J / 2);
             c0[h] = 2 * (I % 2) + 4 * (2 * (J % 2));
-            if (DIM == 3) c0[h] += 4 * 4 * (2 * (K % 2));
             cb[h] = (long long)(fc + cq) * CELLS;
             avg[h] = work && cells_mask[cb[h] + c0[h]] == 1;  // uniform over the NCH lanes of the group
         }
@@ -438,7 +437,6 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const in
             if (avg[h])
 #pragma unroll
                 for (int p = 0; p < Q; p++) fl[h][p] = ST::dec(Fc[(long long)p * ncm + cb[h] + c0[h] + off], (T)VS::w(p));
-        const T scale = (DIM == 2) ? (T)(0.25) : (T)(0.125);
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int ta = ta0 + h * (CELLS / 2);
@@ -447,7 +445,7 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const in
                 const T *f = fl[h];
                 T rho, u, v, w;
                 moments<T, Q>(f, rho, u, v, w);
-                const T udotu = (DIM == 3) ? u * u + v * v + w * w : u * u + v * v;
+                const T udotu = u * u + v * v;
 #pragma unroll
                 for (int p = 0; p < Q; p++) {
                     T cdotu = cdot<T, Q>(p, u, v, w);
@@ -466,7 +464,7 @@ __global__ __launch_bounds__(IWG) void k_avg_interp(FixupArgs<T, S> fa, const in
                 const int p = k + NCH * m;
                 if (avg[h] && p < Q) {
                     const T wq = (T)VelSet<Q>::w(p);
-                    const S enc = ST::enc(scale * acc[m], wq);
+                    const S enc = ST::enc((T)(0.25) * acc[m], wq);
                     Fp[(long long)p * ncm + pcell] = enc;
                     s_avg[p * PPW * CELLS + g * CELLS + ta] = ST::dec(enc, wq);
                 }
@@ -746,83 +744,81 @@ __global__ __launch_bounds__(WG) void k_average(FixupArgs<T, S> fa, const int *_
 {
     using VS = VelSet<Q>;
     if constexpr (FOLD) resolve_pending<T, S, Q>(fa);
-    constexpr int CELLS = VS::CELLS, DIM = VS::DIM;
-    constexpr int NG = (DIM == 3) ? 8 : 4;     // child cells per parent cell
-    constexpr int PER_BLOCK = CELLS / 2 * NG;   // lanes per parent block: two parent cells per lane group
-    __shared__ T s_red[(WG / 64) * Q * 65];     // per-wavefront rows of the group sums
-    if constexpr (DIM == 3) {
+    constexpr int CELLS = VS::CELLS;
+    __shared__ T s_red[(WG / 64) * Q * 65];  // per-wavefront rows of the group sums
+    if constexpr (VS::DIM == 3) {
         const int pb = ids[blockIdx.x], pfc = nbr_child[pb];
         // The same for the whole workgroup.
         if (pfc < 0 || !(ave_type == 2 || blk_mask[pb] == BLK_INTERFACE)) return;
         average_block_3d<T, S, Q>(Fc, ncm, cells_mask, pfc, ave_type, tau_ratio, s_red, [&](int t, int p, T v) {
             Fp[(long long)p * ncm + (long long)pb * CELLS + t] = Store<T, S>::enc(v, (T)VelSet<Q>::w(p));
         });
-        return;
-    }
-    const int k = threadIdx.x % NG;             // which child cell of the group
-    const long long gid = (long long)blockIdx.x * WG + threadIdx.x;
-    const long long bi = gid / PER_BLOCK;
-    const int t0 = (int)((gid % PER_BLOCK) / NG);  // parent cells t0 and t0 + CELLS / 2
-    bool work = bi < n;
-    int b = 0, fc = -1;
-    if (work) {
-        b = ids[bi];
-        fc = nbr_child[b];
-        work = (fc > -1) && (ave_type == 2 || blk_mask[b] == BLK_INTERFACE);
-    }
-    const int off = (k & 1) + 4 * ((k >> 1) & 1) + 16 * ((k >> 2) & 1);
-    bool avg[2];
-    long long ccell[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int t = t0 + h * (CELLS / 2);
-        const int I = t % 4, J = (t / 4) % 4, K = (DIM == 3) ? t / 16 : 0;
-        // Child block of this cell's quadrant and the first cell of its 2x2(x2) group.
-        const int c = (I / 2) + 2 * (J / 2) + 4 * (K / 2);
-        int c0 = 2 * (I % 2) + 4 * (2 * (J % 2));
-        if (DIM == 3) c0 += 4 * 4 * (2 * (K % 2));
-        const long long cb = (long long)(fc + c) * CELLS;
-        avg[h] = false;
+    } else {
+        constexpr int NG = 4;                      // child cells per parent cell
+        constexpr int PER_BLOCK = CELLS / 2 * NG;  // lanes per parent block: two parent cells per lane group
+        const int k = threadIdx.x % NG;            // which child cell of the group
+        const long long gid = (long long)blockIdx.x * WG + threadIdx.x;
+        const long long bi = gid / PER_BLOCK;
+        const int t0 = (int)((gid % PER_BLOCK) / NG);  // parent cells t0 and t0 + CELLS / 2
+        bool work = bi < n;
+        int b = 0, fc = -1;
         if (work) {
-            int m = cells_mask[cb + c0];
-            if (ave_type > 0 && m < 2) m = 1;
-            avg[h] = (m == 1);  // uniform over the NG lanes of the group
+            b = ids[bi];
+            fc = nbr_child[b];
+            work = (fc > -1) && (ave_type == 2 || blk_mask[b] == BLK_INTERFACE);
         }
-        ccell[h] = cb + c0 + off;
-    }
-    T fl[2][Q];
+        const int off = (k & 1) + 4 * (k >> 1);
+        bool avg[2];
+        long long ccell[2];
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-        if (avg[h])
-#pragma unroll
-            for (int p = 0; p < Q; p++) fl[h][p] = Store<T, S>::dec(Fc[(long long)p * ncm + ccell[h]], (T)VS::w(p));
-    const T scale = (DIM == 2) ? (T)(0.25) : (T)(0.125);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        T s[Q];
-        if (avg[h]) {
-            const T *f = fl[h];
-            T rho, u, v, w;
-            moments<T, Q>(f, rho, u, v, w);
-            const T udotu = (DIM == 3) ? u * u + v * v + w * w : u * u + v * v;
-#pragma unroll
-            for (int p = 0; p < Q; p++) {
-                T cdotu = cdot<T, Q>(p, u, v, w);
-                T fe = (T)VS::w(p) * rho * ((T)(1.0) + (T)(3.0) * cdotu + (T)(4.5) * cdotu * cdotu - (T)(1.5) * udotu);
-                s[p] = fe + (f[p] - fe) * tau_ratio;
+        for (int h = 0; h < 2; h++) {
+            const int t = t0 + h * (CELLS / 2);
+            const int I = t % 4, J = t / 4;
+            // Child block of this cell's quadrant and the first cell of its 2x2 group.
+            const int c = (I / 2) + 2 * (J / 2);
+            const int c0 = 2 * (I % 2) + 4 * (2 * (J % 2));
+            const long long cb = (long long)(fc + c) * CELLS;
+            avg[h] = false;
+            if (work) {
+                int m = cells_mask[cb + c0];
+                if (ave_type > 0 && m < 2) m = 1;
+                avg[h] = (m == 1);  // uniform over the NG lanes of the group
             }
-        } else {
-#pragma unroll
-            for (int p = 0; p < Q; p++) s[p] = (T)0;
+            ccell[h] = cb + c0 + off;
         }
-        const long long pcell = (long long)b * CELLS + t0 + h * (CELLS / 2);
-        // s of child cell offsets 0,1,4,5,16,17,20,21 summed left to right (comm.cu:330-339)
-        T acc[(Q + NG - 1) / NG];
-        group_sums<T, Q, NG>(s, acc, s_red + (threadIdx.x >> 6) * Q * 65);
+        T fl[2][Q];
 #pragma unroll
-        for (int m = 0; m < (Q + NG - 1) / NG; m++) {
-            const int p = k + NG * m;
-            if (avg[h] && p < Q) Fp[(long long)p * ncm + pcell] = Store<T, S>::enc(scale * acc[m], (T)VelSet<Q>::w(p));
+        for (int h = 0; h < 2; h++)
+            if (avg[h])
+#pragma unroll
+                for (int p = 0; p < Q; p++) fl[h][p] = Store<T, S>::dec(Fc[(long long)p * ncm + ccell[h]], (T)VS::w(p));
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            T s[Q];
+            if (avg[h]) {
+                const T *f = fl[h];
+                T rho, u, v, w;
+                moments<T, Q>(f, rho, u, v, w);
+                const T udotu = u * u + v * v;
+#pragma unroll
+                for (int p = 0; p < Q; p++) {
+                    T cdotu = cdot<T, Q>(p, u, v, w);
+                    T fe = (T)VS::w(p) * rho * ((T)(1.0) + (T)(3.0) * cdotu + (T)(4.5) * cdotu * cdotu - (T)(1.5) * udotu);
+                    s[p] = fe + (f[p] - fe) * tau_ratio;
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < Q; p++) s[p] = (T)0;
+            }
+            const long long pcell = (long long)b * CELLS + t0 + h * (CELLS / 2);
+            // s of child cell offsets 0,1,4,5 summed left to right (comm.cu:330-339)
+            T acc[(Q + NG - 1) / NG];
+            group_sums<T, Q, NG>(s, acc, s_red + (threadIdx.x >> 6) * Q * 65);
+#pragma unroll
+            for (int m = 0; m < (Q + NG - 1) / NG; m++) {
+                const int p = k + NG * m;
+                if (avg[h] && p < Q) Fp[(long long)p * ncm + pcell] = Store<T, S>::enc((T)(0.25) * acc[m], (T)VelSet<Q>::w(p));
+            }
         }
     }
 }
