@@ -2,7 +2,8 @@
 //
 // HBM layout (all structure-of-arrays, 256-byte aligned allocations):
 //   F[0], F[1]   two population buffers, Q rows x n_maxcells (row q = direction q, physical order);
-//                level L reads F[cur[L]] and writes F[cur[L]^1] in its fused step.
+//                level L reads F[cur[L]] and writes F[cur[L]^1] in its fused step; two sub-steps that
+//                run as an in-place pair stay in F[cur[L]].
 //   M            rho,u,v,w rows x n_maxcells, written only by explicit refresh calls.
 //   cells_mask   n_maxcells ints.
 //   nbr, nbr_child  Q_max rows x n_maxcblocks ints, the reference's velocity-ordered tables
@@ -101,7 +102,8 @@ struct Ctx {
     int *dscal = nullptr;     // small device scalars (counters)
     int *hscal = nullptr;     // pinned host mirror
     // Exceptions of the stream guard: (initiator cell, partner cell, direction) + value, lists of
-    // exc_cap entries: 2L and 2L + 1 of level L, used in turn, and the extra list 2 MAX_LEVELS.
+    // exc_cap entries: 2L and 2L + 1 of level L, used in turn, and the extra list 2 MAX_LEVELS.  With
+    // lists of the largest capacity (2^22 entries, from 65 536 3D blocks on) 64 MiB each, 80 in FP64.
     long long exc_cap = 0, exc_cap_alloc = 0;
     bool exc_overflowed = false;  // an overflow was reported: steps are refused
     int *exc_idx = nullptr;   // 3 ints per entry

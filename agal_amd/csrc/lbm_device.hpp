@@ -114,7 +114,8 @@ constexpr int VMODE_EVEN = 3;
 
 // The memory-side cache.  The first sub-step of an in-place pair reads with ordinary loads when the
 // level's populations fit it (64^3 cavity with three levels, FP32: 288 us a coarse step, 333 with
-// non-temporal ones), else with non-temporal loads (128^3, four levels: 11.9 ms against 11.5).
+// non-temporal ones), else with non-temporal loads (128^3, four levels: 11.5 ms a coarse step, 11.9 with
+// ordinary ones).  Its stores are ordinary ones.
 constexpr long long MALL_BYTES = 256LL << 20;
 
 // Block flag bit: the block has entries in the finest level's extra exception list (bits 0-1 of
@@ -1023,10 +1024,16 @@ __device__ __forceinline__ void fixup_reset(const FixupArgs<T, S> &fa, int lv)
 // last one to pass empties the lists and the counters of this hand-over.  The kernel records into other
 // lists than it resolves here (fold_fixups sees to it), so every workgroup finds the counters as the first
 // did.  Called by all threads of all workgroups, before any exit, in the FOLD variants of the kernels (its mere presence
-// costs a large launch 1-3%).  With entries the hand-over takes 10-15 us, and the
-// acquire of a workgroup that starts later empties the L2 under those that run (64^3 cavity, launches
-// of 6016 workgroups, 130 entries: 547 us a coarse step against 292), so only launches that are bound by
-// their latency do it; the others take a fixup launch before them (fold_fixups).
+// costs a large launch 1-3%).  The line between doing so and a fixup launch before the kernel (fold_fixups)
+// weighs two flows.  With empty lists the hand-over saves about as much at every size, with entries it
+// costs more the larger the launch, because the acquire of a workgroup that starts later empties the L2
+// under those that run.  us per step of one level in D3Q19 FP32, resolved by the step's own kernel / by a fixup launch:
+//   workgroups                                  16           128          250          686          2000         3456
+//   empty lists                                 7.0 / 7.9    7.2 / 8.0    7.6 / 8.4    9.8 / 10.7   18.6 / 19.0  28.4 / 29.1
+//   first eight steps from 2% failing values    12.8 / 12.6  15.3 / 13.0  16.7 / 14.0  22.8 / 16.9  39.0 / 21.6  61 / 44.5
+// (three refined levels, empty lists: 55.5 / 59.4 with launches of up to 160 workgroups, 133 / 135 with 3300).
+// At 128 empty lists, the usual case, save a tenth and entries cost a sixth; beyond, the saving becomes a
+// smaller share of the step and the cost a larger one.
 constexpr int FOLD_MAX_WGS = 128;
 
 template <typename T, typename S, int Q>
@@ -1246,9 +1253,9 @@ static inline int launch_timed(Ctx *c, K kern, int grid, hipStream_t s, double c
 // Two consecutive sub-steps of level L run as an in-place pair where they can: 3D, no linked blocks,
 // every block of the level free of solid cells (its own and its neighbours') with mutual neighbour slots,
 // so that each slot (row, cell) that the second sub-step touches belongs to one cell, and two rows of the
-// pool within 32-bit byte offsets.  us per coarse step, in place with the launch that exchanges the failed
-// links / as fused steps: 64^3 cavity with three levels 286 / 299 in FP32 and 217 / 249 in FP16, one
-// level of 128^3 58.5 / 61.2, 128^3 cavity with four levels 11 650 / 12 200.
+// pool within 32-bit byte offsets.  us per coarse step of D3Q19, in place / as fused steps, all else the same:
+// one level of 36 x 20 x 28 7.0 / 8.4, of 128^3 58.9 / 62.5, 64^3 cavity with three levels 280 / 288 in
+// FP32 and 205 / 213 in FP16, 128^3 cavity with four levels 11 210 / 12 000.
 static inline bool inplace_ok(const Ctx *c, int L)
 {
     return c->DIM == 3 && !c->links_on && L == c->MAX_LEVELS - 1 && c->n_ids[L] > 0 && c->n_general[L] == 0 &&

@@ -72,10 +72,11 @@ __global__ __launch_bounds__(WG) void k_refresh(const int *__restrict__ ids, int
 
 // ---------------------------------------------------------------------------------------------
 // Coarse -> fine: Cu_Interpolate_Linear (solver_lbm_kernels_comm.cu:13-138).  The first CELLS
-// lanes of each parent put the Q rescaled parent populations in LDS; then every lane takes one
-// cell in each half of the children (children c and c + NCH/2), so a parent's children are
-// written by half as many wavefronts with row-contiguous stores.  Half-width groups keep a level's
-// interface parents within one round of resident wavefronts (a 3D parent is one 256-lane
+// lanes of each parent put the Q rescaled parent populations in LDS.  Then the lanes evaluate the
+// children's cells: new children (ADDED) and the plane with one cell per lane in each half of the
+// children (children c and c + NCH/2), row-contiguous stores; interface parents in 3D, where a
+// quarter of the cells are ghost cells, with a list of those (GhostList).  Half-width groups keep a
+// level's interface parents within one round of resident wavefronts (a 3D parent is one 256-lane
 // workgroup; 2D packs eight 4x4 parents).
 // ---------------------------------------------------------------------------------------------
 constexpr int IWG = 256;
@@ -891,7 +892,8 @@ __global__ __launch_bounds__(WG, (COLL == COLL_MRT && Q == 27 && sizeof(T) == 4 
 // Linked blocks (3D, face-cell links of a geometry): the sub-step of blocks holding boundary cells
 // with cut-link fractions.  Cu_Collide, then Cu_ImposeBC with the interpolated bounce-back of
 // Bouzidi, Firdaouss and Lallemand (2001) (solver_lbm_kernels.cu:796-875), then the push of the
-// fused step (push_link), one wavefront per block; the fused step skips these blocks (LINK_FLAG).
+// fused step (push_link), one wavefront per block; the fused step of the same launch skips these blocks
+// (LINK_FLAG, skip_linked).  Where none of the rules is due (link_step_due) the fused step takes them.
 // Both read the level's input buffer and write disjoint slots of its output buffer, and record
 // guard exceptions into the same list, so they can run in either order.
 //

@@ -557,7 +557,8 @@ static int make_bins(Ctx *c)
 }
 
 // The linked blocks of each level (ranked blocks of the level's ID set), concatenated per level,
-// and the LINK_FLAG bit of their block flags (the fused step leaves them to the linked sub-step).
+// and the LINK_FLAG bit of their block flags (the fused step leaves them to the linked sub-step where
+// that is due).
 __global__ void k_link_list_flag(const int *__restrict__ ids, int n, const int *__restrict__ onb_solid,
                                  int *__restrict__ flag)
 {

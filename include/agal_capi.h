@@ -334,7 +334,10 @@ long long agal_load_stl(const char *path, float *out, long long capacity);
  *   nbr, nbr_child: n_q_max arrays of n_blocks ints (velocity-ordered, self at p=0)
  *   per-block ints (ref, level, onb, block mask): n_blocks
  *   coords: n_dim arrays of n_blocks floats
- * `dst_stride` / `src_stride` is the distance in elements between consecutive arrays. */
+ * `dst_stride` / `src_stride` is the distance in elements between consecutive arrays.
+ * Populations and macros of 4 MiB and more go into ordinary (pageable) memory through 16 MiB of pinned
+ * memory that the context's first such download allocates and the context keeps, with three helper
+ * threads during the call. */
 int  agal_download_populations(agal_ctx *ctx, void *dst, long long n_blocks, long long dst_stride);
 int  agal_upload_populations(agal_ctx *ctx, const void *src, long long n_blocks, long long src_stride);
 /* No counterpart in the reference.  agal_download_populations for callers that cannot allocate
@@ -393,13 +396,13 @@ int  agal_import_pool(agal_ctx *ctx, const agal_pool *pool);
  * and BF16 pools) on matrix cores: per block, (moments x directions) . (directions x 64 cells)
  * products in v_mfma_f32_16x16x32_bf16 with the non-equilibrium parts and the relaxed moments
  * split into two bf16 terms (16 significant bits of a small correction; FP32 sums in the hardware's
- * order).  0 (default) keeps the vector path, whose sums follow a fixed order shared with the CPU
- * restatement. */
+ * order).  Blocks with face-cell links keep the vector path.  0 (default) keeps it for all blocks: its
+ * sums follow a fixed order shared with the CPU restatement. */
 #define AGAL_OPT_MRT_MFMA 2
 /* AGAL_OPT_EXC_CAP: entries per stream-guard exception list (default and maximum:
- * min(cells of the pool, 2^22) per level).  A sub-step whose list overflows drops links; the next
- * agal_sync / agal_advance_loop reports AGAL_ERR_OVERFLOW and the context refuses further steps
- * (AGAL_ERR_STATE). */
+ * min(cells of the pool, 2^22) per list, two lists per level and one more).  A sub-step whose list
+ * overflows drops links; the next agal_sync / agal_advance_loop reports AGAL_ERR_OVERFLOW and the
+ * context refuses further steps (AGAL_ERR_STATE). */
 #define AGAL_OPT_EXC_CAP 3
 /* AGAL_OPT_GRAPH_STEPS: coarse steps of agal_advance_loop recorded into one graph at most (1..64,
  * default 4).  Longer graphs amortize the gap between graph launches; each distinct length is a
